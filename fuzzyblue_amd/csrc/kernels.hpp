@@ -104,21 +104,48 @@ constexpr int kSsTexelsPerThread = 4;
 constexpr size_t kDenSplitTexels = 65536;
 // Density texels per thread: 2 when the LUT set is not theta-split, NU is
 // even and an (r, mu_s) tile holds at least kDenPairMinTexels texels — the
-// thread then takes texels (mu, nu) and (mu, nu + NU/2), which share
-// nu2 = omega.omega_i, q and the Cornette-Shanks power of every direction
-// pair (computed once for both; each texel's own operations and their order
-// are unchanged, so the values are the same bits), and a block's profile
-// build serves twice the texels.
+// thread then takes texels (mu, nu index k) and (mu, NU-1-k), which share
+// nu2 = omega.omega_i and the phase weight of every direction pair (computed
+// once for both), and a block's profile build serves twice the texels.
 constexpr int kDenPairMinTexels = 512;
-// Blocks per CU the density kernels are compiled for: 8 at one texel per
-// thread (64 VGPRs), 5 at two (91-96).  Four texels per thread (3 blocks,
-// 138-143 VGPRs) measured 6% slower at double and 30% at default sizes; at
-// two, 4 blocks for order 2 (no spills) was 1% slower than 5.
-__host__ __device__ constexpr int den_occupancy(int tpx, bool) { return tpx == 1 ? 8 : 5; }
-__host__ __device__ inline int den_tpx(const DevParams& P) {
-    return (P.den_split == 1 && P.s_nu % 2 == 0 && P.s_mu * P.s_nu >= kDenPairMinTexels) ? 2
-                                                                                          : 1;
+// Blocks per CU the density kernels are compiled for.  One texel per thread:
+// 4 (8 blocks, 64 VGPRs, spill: 0.066 instead of 0.041 ms per order >= 3
+// launch of a half-resolution set, whose blocks do not fill the chip).  Two:
+// 6 at order >= 3 (5: 2.69 instead of 2.60 ms at double), 5 at order 2 (6:
+// 5.30 instead of 5.23 ms).
+__host__ __device__ constexpr int den_occupancy(int tpx, bool single) {
+    return tpx == 1 ? 4 : (single ? 5 : 6);
 }
+// Whether the density pass runs the outer texels (nu index 0 and NU-1) on
+// their shortcut: precision mode.  FP32 mode follows the reference's
+// binary32 omega_s, which is off the meridian plane by its rounding, lookup
+// by lookup (with the shortcut one texel in 10^5 is 1e-4 from it).
+__host__ __device__ inline bool den_outer(const DevParams& P) { return P.flags & 1; }
+__host__ __device__ inline int den_tpx(const DevParams& P) {
+    return (P.den_split == 1 && (P.s_nu > 2 || !den_outer(P)) && P.s_nu % 2 == 0 &&
+            P.s_mu * P.s_nu >= kDenPairMinTexels)
+               ? 2
+               : 1;
+}
+// Row stride of the density kernel's table of outer incident radiance: 16
+// entries and one pad, so that the lanes of a theta-split group, each on its
+// own row, read from different banks.
+constexpr int kDenOuterStride = kDenPhi / 2 + 1;
+// The threads of one (r, mu_s) tile of the density pass: [0, inner) take the
+// texels of nu index first..NU-1-first (groups x threads per group, rounded
+// up to whole wavefronts), [inner, total) the outer ones (nu index 0 and
+// NU-1, where they have a path of their own: first = 1), both of one mu per
+// thread group.
+struct DenLayout {
+    int first, groups, inner, total;
+    __host__ __device__ DenLayout(const DevParams& P, int tpx) {
+        const int split = tpx > 1 ? 1 : P.den_split;
+        first = den_outer(P) ? 1 : 0;
+        groups = P.s_mu * (P.s_nu - 2 * first) / tpx;
+        inner = (groups * split + 63) / 64 * 64;
+        total = inner + first * P.s_mu * split;
+    }
+};
 constexpr int kSsMaxStagedMu = 2048;
 // Multiple scattering over rows of at most kMsChunkMaxW texels (small LUT
 // sets, whose launches are a few hundred one-wavefront blocks, each walking
