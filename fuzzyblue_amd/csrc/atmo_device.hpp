@@ -23,9 +23,15 @@ struct DevLayer {
     float width, exp_term, exp_scale, linear_term, constant_term;
 };
 
+// Constants of the multiple-scattering samples' mu_s coordinate (MsCoord),
+// evaluated in binary64 by the host.
+struct MsCoordConst {
+    float c, c2, p0, p1, q0;
+};
+
 // Mirrors shaders/params.h:26-87 (AtmosphereParameters), field for field,
-// plus the texture sizes.  Passed by value as a kernel argument (252 B) or
-// read from an HBM array in the batched passes.
+// plus the texture sizes and derived constants.  Passed by value as a kernel
+// argument (272 B) or read from an HBM array in the batched passes.
 struct DevParams {
     float solar[3];
     float sun_angular_radius;
@@ -42,6 +48,7 @@ struct DevParams {
     int t_mu, t_r, s_r, s_mu, s_mus, s_nu, i_mus, i_r;
     int den_split;        // scattering density: threads per texel (1, or kDenTheta)
     DevLayer prof[3][2];  // rayleigh, mie, absorption
+    MsCoordConst ms;
 };
 
 constexpr float kPi = 3.14159265358979323846f;

@@ -398,7 +398,8 @@ __device__ __forceinline__ void row_geometry_block(const DevParams& P, const int
     const MsSlots sl = ms_row_slots(i, tz4, ty4, off, wt);
     if (!writer) return;
     m[i] = make_float4(tv.x * f, tv.y * f, tv.z * f, float(d_i));
-    m[kMsSamples + i] = make_float4(float(G(1) / r_d), __int_as_float(sl.mask), 0.0f, 0.0f);
+    m[kMsSamples + i] =
+        make_float4(float(r / r_d), __int_as_float(sl.mask), float(d_i / r_d), 0.0f);
     reinterpret_cast<int4*>(m + 2 * kMsSamples)[i] = sl.load;
     m[3 * kMsSamples + i] = sl.w;
 }
@@ -1518,10 +1519,19 @@ __device__ __forceinline__ void indirect_irradiance_block(const DevParams& P, co
 // All texels of one (r, mu) row (x = nu*MUS + mu_s varies) march the same
 // ray: d_i, r_i, mu_i, the view transmittance T(r, mu, d_i) and the
 // (u_mu, u_r) taps of every sample are shared, only mu_s_i (and the fixed
-// nu slice) differ per texel.  A block owns one row: it computes the 51
-// sample descriptors once, and for each sample stages the (mu, r)-bilinear
-// row of the density LUT in LDS (double buffered, one barrier per sample);
-// each texel then lerps 2 nu slices x 2 mu_s taps from LDS.
+// nu slice) differ per texel.  A block owns one row: for each sample it
+// stages the (mu, r)-bilinear row of the density LUT in LDS (double buffered,
+// one barrier per sample), and each texel lerps its mu_s taps from LDS: two
+// in its own nu slice, and two in the next where its nu falls between slices
+// (MsTexel).
+//
+// Where the density LUT fits the L2s it is bound by the chain of a sample
+// (coordinate, LDS taps, staging, barrier), else by the latency of the row
+// loads that miss the L2 (10 GB from beyond it per launch at double).  With
+// four taps for every texel and the coordinate after the barrier a launch took
+// 0.118 ms at default and 0.149 at 27x64x26x18, now 0.097 and 0.087; at double
+// 2.35, now 2.21.  Loads two samples ahead (24 more VGPRs): 2.48 at double,
+// 0.123 at default.
 constexpr int kMsTexelsPerThread = 4;
 // Threads per block of the multiple-scattering kernels: up to one per
 // texel of the widest row (NU * MUS <= 1024).
@@ -1541,10 +1551,97 @@ __device__ __forceinline__ Rgb to_rgb(const Half4& v) {
     return Rgb{float(v.x), float(v.y), float(v.z)};
 }
 
+// GetScatteringTextureUvwzFromRMuMuSNu's mu_s coordinate (scattering.h:
+// 48-56) of a sample, (1 - a/A) / (1 + a) (MUS-1), as the texel coordinate
+// within a nu slice.  a = (d - d_min) / (d_max - d_min), d the distance from
+// the ground to the top boundary at mu_s, d / H = sqrt(c^2 mu_s^2 + 1) - c
+// mu_s, c = bottom / H.  With u = sqrt(c^2 mu_s^2 + 1) + c |mu_s|, which has
+// no cancellation, d / H is u for mu_s < 0 and 1 / u otherwise, and the
+// coordinate is a quotient of two linear functions of it: three times closer
+// to the exact coordinate than the difference of two terms of bottom's size.
+// Kept in [0, MUS-1] (a >= 0 up to rounding, and the reference clamps 1 - a/A
+// at 0).  FP32 mode takes the reference's expression.
+template <typename G>
+struct MsCoord {
+    MsCoordConst k;
+    float top;
+    __device__ explicit MsCoord(const DevParams& P) : k(P.ms), top(float(P.s_mus - 1)) {}
+    // mu_s at the sample (multiple_scattering.comp:38): (r mu_s + d_i nu) / r_i.
+    __device__ float operator()(float mu_s, float nu, float r_ri, float d_ri) const {
+        const float m = fmaf(r_ri, mu_s, d_ri * nu);
+        const float u = fmaf(k.c, fabsf(m), __builtin_amdgcn_sqrtf(fmaf(k.c2, m * m, 1.0f)));
+        const float s = m < 0.0f ? u : 1.0f, t = m < 0.0f ? 1.0f : u;
+        return __builtin_amdgcn_fmed3f(
+            fmaf(k.p1, s, k.p0 * t) * __builtin_amdgcn_rcpf(fmaf(k.q0, t, s)), 0.0f, top);
+    }
+};
+template <>
+struct MsCoord<float> {
+    float b, b2, h2, d_min, inv, inv_a, top;
+    __device__ explicit MsCoord(const DevParams& P) {
+        b = P.bottom;
+        b2 = b * b;
+        h2 = P.top * P.top - b2;
+        d_min = P.top - b;
+        inv = 1.0f / (sqrtf(h2) - d_min);
+        inv_a = 1.0f / (-2.0f * P.mu_s_min * b * inv);
+        top = float(P.s_mus - 1);
+    }
+    __device__ float operator()(float mu_s, float nu, float r_ri, float d_ri) const {
+        const float m = __builtin_amdgcn_fmed3f(fmaf(r_ri, mu_s, d_ri * nu), -1.0f, 1.0f);
+        const float d =
+            fmaxf(fmaf(-b, m, __builtin_amdgcn_sqrtf(fmaf(b2, m * m, h2))), 0.0f);
+        const float a = (d - d_min) * inv;
+        return top * __builtin_amdgcn_fmed3f(
+                         fmaf(-a, inv_a, 1.0f) * __builtin_amdgcn_rcpf(1.0f + a), 0.0f, 1.0f);
+    }
+};
+
+// A row's texels in thread order.  Position x of the row is nu slot x / MUS:
+// nu index 0, NU-1, 1, 2, ..., NU-2, so that the outer texels come first.
+__device__ __forceinline__ int ms_nu_index(int slot, int NU) {
+    return slot == 0 ? 0 : (slot == 1 ? NU - 1 : slot - 1);
+}
+
+// A texel of a multiple-scattering row.  nu is constant along the ray, so an
+// inner texel, whose nu is its slice's, reads that slice only (lerp 0); where
+// nu is clamped (scattering.h:132-134) it falls between slices.  An inner
+// index with a clamped nu has the nu, mu_s and so the value of the outer texel
+// on its side: its thread copies that one's sum (`copy`: 1 + 0 for index 0's,
+// 1 + 1 for NU-1's, 0 if the texel has a value of its own).  FP32 mode, where
+// mu_s depends on the nu index by its rounding, evaluates it like an outer one.
+struct MsTexel {
+    float mu_s, nu, lerp;
+    int x, entry, copy;  // x: texel in the row; entry: slice's first staged entry
+    bool two;            // reads two slices
+};
+template <typename G>
+__device__ __forceinline__ MsTexel ms_texel(const DevParams& P, int slot, int j, int y, int z) {
+    const int NU = P.s_nu, k = ms_nu_index(slot, NU);
+    MsTexel t;
+    t.x = k * P.s_mus + j;
+    const TexelCoord<G> c = scattering_texel_coord<G>(P, unsigned(t.x), unsigned(y), unsigned(z));
+    t.mu_s = float(c.mu_s);
+    t.nu = float(c.nu);
+    const G knot = clamp_cosine<G>(G(k) / G(NU - 1) * G(2) - G(1));  // as in the texel map
+    const float tc = (t.nu + 1.0f) / 2.0f * float(NU - 1);
+    float slice = floorf(tc);
+    t.lerp = tc - slice;
+    t.copy = 0;
+    t.two = slot < 2 || (c.nu != knot && sizeof(G) == sizeof(float));
+    if (!t.two) {
+        slice = float(k);
+        t.lerp = 0.0f;
+        if (c.nu != knot) t.copy = c.nu > knot ? 1 : 2;
+    }
+    t.entry = int(slice) * (P.s_mus + 1);
+    return t;
+}
+
 // H: the density LUT J, the delta and the scattering LUT are binary16
 // (FB_FLAG_F16_STORAGE); the density rows then stay binary16 in the slots
 // until put() widens them.
-template <typename G, bool COMP, int TPT, bool H>
+template <typename G, int TPT, bool H>
 __device__ __forceinline__ void multiple_scattering_block(const DevParams& P, const int bx, const int by, const int bz,
                                                              const float4* __restrict__ MR,
                                                              const float4* __restrict__ J,
@@ -1564,51 +1661,32 @@ __device__ __forceinline__ void multiple_scattering_block(const DevParams& P, co
     typedef FB_CONSTANT_AS const int4 CI4;
     CF4* desc = (CF4*)(MR + (size_t(z) * MU + y) * kMsRowFloat4s);
     auto d_tw = [&](int i) { return desc[i]; };  // T(r,mu,d_i)*dx*weight (rgb), d_i
-    auto d_geo = [&](int i) { return desc[kMsSamples + i]; };  // 1/r_i, slot load mask
+    auto d_geo = [&](int i) { return desc[kMsSamples + i]; };  // r/r_i, slot load mask, d_i/r_i
     auto d_off = [&](int i) { return ((CI4*)(desc + 2 * kMsSamples))[i]; };  // slot rows
     auto d_wt = [&](int i) { return desc[3 * kMsSamples + i]; };  // slot weights
-    const G r = scattering_texel_coord<G>(P, 0u, unsigned(y), unsigned(z)).r;
 
-    // Per-texel constants: mu_s, nu, nu slice and its lerp weight.
-    float tmu_s[TPT], tnu[TPT], tslice[TPT], tlerp[TPT];
-    int spos[TPT];  // the texel's entry in a staged row
-    Sum<COMP> acc[TPT][3];
-    const float rf = float(r);
+    // Per-texel constants: thread tid's texels are positions tid + q*nt.
+    MsTexel tx[TPT];
+    bool inner[TPT];  // every texel of the wavefront reads one slice (wave-uniform)
+    int spos[TPT];    // the texel's entry in a staged row
+    float acc0[TPT], acc1[TPT], acc2[TPT];
 #pragma unroll
     for (int q = 0; q < TPT; ++q) {
         const int x = tid + q * nt;
-        tmu_s[q] = 0.0f;
-        tnu[q] = 0.0f;
-        tslice[q] = 0.0f;
-        tlerp[q] = 0.0f;
-        spos[q] = x + x / MUS;
-        if (x < W) {
-            TexelCoord<G> c = scattering_texel_coord<G>(P, unsigned(x), unsigned(y), unsigned(z));
-            tmu_s[q] = float(c.mu_s);
-            tnu[q] = float(c.nu);
-            float u_nu = (tnu[q] + 1.0f) / 2.0f;
-            float tcx = u_nu * float(NU - 1);
-            tslice[q] = floorf(tcx);
-            tlerp[q] = tcx - tslice[q];
-        }
+        tx[q] = MsTexel{0.0f, 0.0f, 0.0f, 0, 0, 0, false};
+        if (x < W) tx[q] = ms_texel<G>(P, x / MUS, x % MUS, y, z);
+        inner[q] = __builtin_amdgcn_ballot_w64(tx[q].two) == 0;
+        spos[q] = tx[q].x + tx[q].x / MUS;
+        acc0[q] = acc1[q] = acc2[q] = 0.0f;
     }
     __syncthreads();
 
-    // GetScatteringTextureUvwzFromRMuMuSNu's mu_s coordinate (scattering.h:
-    // 48-56) folded into the texel coordinate of slice `tslice`:
-    // x_tex = x_mu_s*(MUS-1) + tslice*MUS, with reciprocals hoisted; in a
-    // staged row, slice k starts at entry k*(MUS + 1).
-    const float b = P.bottom, b2 = P.bottom * P.bottom;
-    const float H2 = P.top * P.top - P.bottom * P.bottom;
-    const float d_min = P.top - P.bottom;
-    const float inv_range = 1.0f / (sqrtf(H2) - d_min);
-    const float invA = 1.0f / (-2.0f * P.mu_s_min * P.bottom * inv_range);
-    const int SS = MUS + 1;
-    const float musm1 = float(MUS - 1), fSS = float(SS);
+    const MsCoord<G> coord(P);
+    const int SS = MUS + 1;  // staged entries per nu slice
 
-    // The four density-row slots of this thread's texels x = tid + q*nt,
-    // carried from sample to sample (ms_row_slots): each sample loads only
-    // the rows it does not share with the previous one.
+    // The four density-row slots of this thread's texels, carried from sample
+    // to sample (ms_row_slots): each sample loads only the rows it does not
+    // share with the previous one.
     typedef typename std::conditional<H, Half4, Rgb>::type Slot;
     Slot slot[TPT][4];
 #pragma unroll
@@ -1618,13 +1696,13 @@ __device__ __forceinline__ void multiple_scattering_block(const DevParams& P, co
     // Row loads as buffer loads: the row start (block-uniform) goes in the
     // scalar offset and the texel's byte offset in a loop-invariant vector
     // offset, so no address arithmetic writes a register between the loads
-    // and each load lands directly in its slot.  Loads past the LUT's end
-    // (texels x >= W of the last row) return 0 and are never used.
+    // and each load lands directly in its slot.  (Positions past the row load
+    // texel 0 and never use it.)
     constexpr int TB = H ? 8 : 16;  // bytes per texel of J
     const __amdgpu_buffer_rsrc_t jb = buffer_rsrc(J, int(size_t(P.s_r) * MU * W * TB));
     int xoff[TPT];
 #pragma unroll
-    for (int q = 0; q < TPT; ++q) xoff[q] = (tid + q * nt) * TB;
+    for (int q = 0; q < TPT; ++q) xoff[q] = tx[q].x * TB;
     auto ld = [&](int o, int q) {
         if constexpr (H) {
             return __builtin_bit_cast(Half4,
@@ -1673,73 +1751,86 @@ __device__ __forceinline__ void multiple_scattering_block(const DevParams& P, co
         for (int q = 0; q < TPT; ++q)
             if (tid + q * nt < W) put(i, slot[q], dst, spos[q]);
     };
-    // Sample i of every texel of this thread, from the staged row `cur`.
-    auto eval = [&](int i, const Rgb* __restrict__ cur) {
-        const float4 tw = d_tw(i);
-        const float inv_r_i = d_geo(i).x, d_i = tw.w;
+    // A texel's mu_s coordinate at sample i, and sample i of every texel of
+    // this thread from the staged row `cur`: the coordinates of sample i+1
+    // are computed while the taps of sample i are on their way from LDS.
+    float xt[TPT];
+    auto locate = [&](float4 geo, int q) {
+        return coord(tx[q].mu_s, tx[q].nu, geo.x, geo.z);
+    };
+    auto eval = [&](float4 tw, float4 geo_next, const Rgb* __restrict__ cur) {
 #pragma unroll
         for (int q = 0; q < TPT; ++q) {
-            const int x = tid + q * nt;
-            if (x < W) {
-                // mu_s at the sample (multiple_scattering.comp:38), in [-1, 1].
-                float mu_s_i = fmaf(rf, tmu_s[q], d_i * tnu[q]) * inv_r_i;
-                mu_s_i = __builtin_amdgcn_fmed3f(mu_s_i, -1.0f, 1.0f);
-                float disc = fmaf(b2, mu_s_i * mu_s_i, H2);
-                float d = fmaxf(fmaf(-b, mu_s_i, __builtin_amdgcn_sqrtf(disc)), 0.0f);
-                float a = (d - d_min) * inv_range;
-                // max(1 - a/A, 0) / (1 + a), kept <= 1 (a >= 0 up to rounding).
-                float xm = __builtin_amdgcn_fmed3f(
-                    fmaf(-a, invA, 1.0f) * __builtin_amdgcn_rcpf(1.0f + a), 0.0f, 1.0f);
-                float xt = fmaf(xm, musm1, tslice[q] * fSS);
-                float fl = floorf(xt);
-                float w = xt - fl;
-                int i0 = int(fl);
-                // 0 <= i0 - tslice*SS <= MUS - 1 (0 <= xm <= 1, 0 <= tslice
-                // <= NU - 1): the taps i0, i0+1, i0+SS, i0+SS+1 stay inside
-                // the padded row (see the layout above).
-                const Rgb p0 = cur[i0], p1 = cur[i0 + 1], p2 = cur[i0 + SS],
-                          p3 = cur[i0 + SS + 1];
-                float l = tlerp[q];
+            if (tid + q * nt < W) {
+                // 0 <= xt <= MUS - 1 and 0 <= entry <= (NU - 1) SS: the taps
+                // i0, i0+1, i0+SS, i0+SS+1 stay inside the padded row (see the
+                // layout above).
+                const float w = __builtin_amdgcn_fractf(xt[q]);
+                const Rgb* p = cur + (tx[q].entry + int(xt[q]));
+                const Rgb p0 = p[0], p1 = p[1];
+                xt[q] = locate(geo_next, q);
                 float v0 = fmaf(w, p1.x - p0.x, p0.x), v1 = fmaf(w, p1.y - p0.y, p0.y),
                       v2 = fmaf(w, p1.z - p0.z, p0.z);
-                float u0 = fmaf(w, p3.x - p2.x, p2.x), u1 = fmaf(w, p3.y - p2.y, p2.y),
-                      u2 = fmaf(w, p3.z - p2.z, p2.z);
-                acc[q][0].add(fmaf(l, u0 - v0, v0) * tw.x);
-                acc[q][1].add(fmaf(l, u1 - v1, v1) * tw.y);
-                acc[q][2].add(fmaf(l, u2 - v2, v2) * tw.z);
+                if (!inner[q]) {
+                    const Rgb p2 = p[SS], p3 = p[SS + 1];
+                    const float u0 = fmaf(w, p3.x - p2.x, p2.x), u1 = fmaf(w, p3.y - p2.y, p2.y),
+                                u2 = fmaf(w, p3.z - p2.z, p2.z);
+                    const float l = tx[q].lerp;
+                    v0 = fmaf(l, u0 - v0, v0);
+                    v1 = fmaf(l, u1 - v1, v1);
+                    v2 = fmaf(l, u2 - v2, v2);
+                }
+                acc0[q] = fmaf(v0, tw.x, acc0[q]);
+                acc1[q] = fmaf(v1, tw.y, acc1[q]);
+                acc2[q] = fmaf(v2, tw.z, acc2[q]);
             }
         }
     };
-    // (Each thread stages exactly its own texels x = tid + q*nt: W <= TPT*nt.)
-    advance(__float_as_int(d_geo(0).y), d_off(0));
+    // (Each thread stages exactly its own texels: W <= TPT*nt.)
+    float4 geo = d_geo(0);
+    advance(__float_as_int(geo.y), d_off(0));
     put_all(0, s_row);
+#pragma unroll
+    for (int q = 0; q < TPT; ++q) xt[q] = locate(geo, q);
     __syncthreads();
-    // The slot mask and row offsets of the sample after next are read (scalar
-    // loads) one iteration ahead of their use.
-    int mask_n = __float_as_int(d_geo(1).y);
-    int4 o_n = d_off(1);
+    // The descriptors of the sample after next are read (scalar loads) one
+    // iteration ahead of their use.
+    geo = d_geo(1);
+    int4 off = d_off(1);
     for (int i = 0; i < kMsSamples; ++i) {
         const Rgb* cur = s_row + (i & 1) * WP;
         Rgb* nxt = s_row + ((i + 1) & 1) * WP;
         const bool next = i + 1 < kMsSamples;
         // The loads of sample i+1 are issued first, so that their latency
         // overlaps the evaluation of sample i.
-        if (next) advance(mask_n, o_n);
+        if (next) advance(__float_as_int(geo.y), off);
         const int i2 = i + 2 < kMsSamples ? i + 2 : kMsSamples - 1;
-        mask_n = __float_as_int(d_geo(i2).y);
-        o_n = d_off(i2);
-        eval(i, cur);
+        const float4 geo2 = d_geo(i2);
+        off = d_off(i2);
+        eval(d_tw(i), geo, cur);
         if (next) put_all(i + 1, nxt);
         __syncthreads();
+        geo = geo2;
     }
+    // The outer texels' sums (positions 0..2 MUS-1), for the threads that
+    // copy them.
+#pragma unroll
+    for (int q = 0; q < TPT; ++q)
+        if (tid + q * nt < 2 * MUS) s_row[tid + q * nt] = Rgb{acc0[q], acc1[q], acc2[q]};
+    __syncthreads();
 #pragma unroll
     for (int q = 0; q < TPT; ++q) {
-        const int x = tid + q * nt;
-        if (x < W) {
-            const size_t idx = (size_t(z) * MU + y) * W + x;
-            float m0 = acc[q][0].value(), m1 = acc[q][1].value(), m2 = acc[q][2].value();
+        if (tid + q * nt < W) {
+            const size_t idx = (size_t(z) * MU + y) * W + tx[q].x;
+            float m0 = acc0[q], m1 = acc1[q], m2 = acc2[q];
+            if (tx[q].copy) {
+                const Rgb o = s_row[(tx[q].copy - 1) * MUS + tx[q].x % MUS];
+                m0 = o.x;
+                m1 = o.y;
+                m2 = o.z;
+            }
             st_tex(dMS, idx, make_float4(m0, m1, m2, 0.0f), H);
-            float pr = phase_rayleigh(tnu[q]);
+            float pr = phase_rayleigh(tx[q].nu);
             float4 prev = ld_tex(S, idx, H);
             st_tex(S, idx,
                    make_float4(m0 / pr + prev.x, m1 / pr + prev.y, m2 / pr + prev.z,
@@ -1783,8 +1874,6 @@ __device__ __forceinline__ void multiple_scattering_block_chunked(
     auto d_geo = [&](int i) { return s_desc[kMsSamples + i]; };
     auto d_off = [&](int i) { return reinterpret_cast<const int4*>(s_desc + 2 * kMsSamples)[i]; };
     auto d_wt = [&](int i) { return s_desc[3 * kMsSamples + i]; };
-    const G r = scattering_texel_coord<G>(P, 0u, unsigned(y), unsigned(z)).r;
-    const float rf = float(r);
 
     float tmu_s = 0.0f, tnu = 0.0f, tslice = 0.0f, tlerp = 0.0f;
     if (in_chunk) {
@@ -1798,13 +1887,9 @@ __device__ __forceinline__ void multiple_scattering_block_chunked(
     }
     const int spos = x + x / MUS;
 
-    const float b = P.bottom, b2 = P.bottom * P.bottom;
-    const float H2 = P.top * P.top - P.bottom * P.bottom;
-    const float d_min = P.top - P.bottom;
-    const float inv_range = 1.0f / (sqrtf(H2) - d_min);
-    const float invA = 1.0f / (-2.0f * P.mu_s_min * P.bottom * inv_range);
+    const MsCoord<G> coord(P);
     const int SS = MUS + 1;
-    const float musm1 = float(MUS - 1), fSS = float(SS);
+    const int entry = int(tslice) * SS;
 
     typedef typename std::conditional<H, Half4, Rgb>::type Slot;
     Slot slot[4];
@@ -1847,28 +1932,19 @@ __device__ __forceinline__ void multiple_scattering_block_chunked(
     };
     float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
     auto eval = [&](int i, const Rgb* __restrict__ cur) {
-        const float4 tw = d_tw(i);
-        const float inv_r_i = d_geo(i).x, d_i = tw.w;
-        float mu_s_i = fmaf(rf, tmu_s, d_i * tnu) * inv_r_i;
-        mu_s_i = __builtin_amdgcn_fmed3f(mu_s_i, -1.0f, 1.0f);
-        float disc = fmaf(b2, mu_s_i * mu_s_i, H2);
-        float d = fmaxf(fmaf(-b, mu_s_i, __builtin_amdgcn_sqrtf(disc)), 0.0f);
-        float a = (d - d_min) * inv_range;
-        float xm = __builtin_amdgcn_fmed3f(
-            fmaf(-a, invA, 1.0f) * __builtin_amdgcn_rcpf(1.0f + a), 0.0f, 1.0f);
-        float xt = fmaf(xm, musm1, tslice * fSS);
-        float fl = floorf(xt);
-        float w = xt - fl;
-        int k0 = int(fl);
+        const float4 tw = d_tw(i), geo = d_geo(i);
+        const float xt = coord(tmu_s, tnu, geo.x, geo.z);
+        const float w = __builtin_amdgcn_fractf(xt);
+        const int k0 = entry + int(xt);
         const Rgb p0 = cur[k0], p1 = cur[k0 + 1], p2 = cur[k0 + SS], p3 = cur[k0 + SS + 1];
         float l = tlerp;
         float v0 = fmaf(w, p1.x - p0.x, p0.x), v1 = fmaf(w, p1.y - p0.y, p0.y),
               v2 = fmaf(w, p1.z - p0.z, p0.z);
         float u0 = fmaf(w, p3.x - p2.x, p2.x), u1 = fmaf(w, p3.y - p2.y, p2.y),
               u2 = fmaf(w, p3.z - p2.z, p2.z);
-        a0 = a0 + fmaf(l, u0 - v0, v0) * tw.x;
-        a1 = a1 + fmaf(l, u1 - v1, v1) * tw.y;
-        a2 = a2 + fmaf(l, u2 - v2, v2) * tw.z;
+        a0 = fmaf(fmaf(l, u0 - v0, v0), tw.x, a0);
+        a1 = fmaf(fmaf(l, u1 - v1, v1), tw.y, a1);
+        a2 = fmaf(fmaf(l, u2 - v2, v2), tw.z, a2);
     };
     __syncthreads();  // the table and the rows' pads
     // The rows the four slots hold at each sample: a slot that a sample uses
@@ -2155,7 +2231,7 @@ __global__ __launch_bounds__(64 * kIndWaves) void kb_indirect_irradiance(
     }
 }
 
-template <typename G, bool COMP, int TPT, bool H>
+template <typename G, int TPT, bool H>
 __global__ __launch_bounds__(kMsMaxThreads) void k_multiple_scattering(DevParams P,
                                                              const float4* __restrict__ MR,
                                                              const float4* __restrict__ J,
@@ -2163,9 +2239,9 @@ __global__ __launch_bounds__(kMsMaxThreads) void k_multiple_scattering(DevParams
                                                              float4* __restrict__ S,
                                                              unsigned remap) {
     const unsigned b = logical_block(remap);
-    multiple_scattering_block<G, COMP, TPT, H>(P, b % P.s_mu, b / P.s_mu, 0, MR, J, dMS, S);
+    multiple_scattering_block<G, TPT, H>(P, b % P.s_mu, b / P.s_mu, 0, MR, J, dMS, S);
 }
-template <typename G, bool COMP, int TPT, bool H>
+template <typename G, int TPT, bool H>
 __global__ __launch_bounds__(kMsMaxThreads) void kb_multiple_scattering(const DevParams* __restrict__ Ps,
                                                               const LutPtrs* __restrict__ L,
                                                               const uint32_t* __restrict__ tiles, unsigned ntiles) {
@@ -2178,7 +2254,7 @@ __global__ __launch_bounds__(kMsMaxThreads) void kb_multiple_scattering(const De
         decode_tile(tiles[t], atm, local);
         const DevParams& P = Ps[atm];
         const LutPtrs l = lut_ptrs(L, atm);
-        multiple_scattering_block<G, COMP, TPT, H>(P, local % P.s_mu, local / P.s_mu, 0, l.MR,
+        multiple_scattering_block<G, TPT, H>(P, local % P.s_mu, local / P.s_mu, 0, l.MR,
                                                    l.J, l.dMS, l.S);
     }
 }
@@ -2396,7 +2472,7 @@ static hipError_t launch_multiple_scattering_h(const DevParams& P, const float4*
     const int tpt = W <= threads ? 1 : (W <= 2 * threads ? 2 : 4);
     const bool precise = P.flags & 1;
 #define FB_MS(G, TPT) \
-    k_multiple_scattering<G, false, TPT, H><<<grid, threads, lds, s>>>(P, MR, J, dMS, S, remap)
+    k_multiple_scattering<G, TPT, H><<<grid, threads, lds, s>>>(P, MR, J, dMS, S, remap)
     if (precise)
         tpt == 1 ? FB_MS(double, 1) : tpt == 2 ? FB_MS(double, 2) : FB_MS(double, 4);
     else
@@ -2576,7 +2652,7 @@ static hipError_t launch_batch_h(int pass, int order, bool precise, const DevPar
                 kb_indirect_irradiance<float, false, H><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles);
             break;
         case kPassMultiple:
-#define FB_KBMS(G, T) kb_multiple_scattering<G, false, T, H><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles)
+#define FB_KBMS(G, T) kb_multiple_scattering<G, T, H><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles)
             if (tpt == kMsChunkedTpt) {
                 if (precise)
                     kb_multiple_scattering_chunked<double, H><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles);
@@ -2659,14 +2735,14 @@ static unsigned batch_resident_blocks_h(int pass, int order, bool precise, unsig
                 fn = precise ? (const void*)kb_multiple_scattering_chunked<double, H>
                              : (const void*)kb_multiple_scattering_chunked<float, H>;
             else if (tpt == 1)
-                fn = precise ? (const void*)kb_multiple_scattering<double, false, 1, H>
-                             : (const void*)kb_multiple_scattering<float, false, 1, H>;
+                fn = precise ? (const void*)kb_multiple_scattering<double, 1, H>
+                             : (const void*)kb_multiple_scattering<float, 1, H>;
             else if (tpt == 2)
-                fn = precise ? (const void*)kb_multiple_scattering<double, false, 2, H>
-                             : (const void*)kb_multiple_scattering<float, false, 2, H>;
+                fn = precise ? (const void*)kb_multiple_scattering<double, 2, H>
+                             : (const void*)kb_multiple_scattering<float, 2, H>;
             else
-                fn = precise ? (const void*)kb_multiple_scattering<double, false, 4, H>
-                             : (const void*)kb_multiple_scattering<float, false, 4, H>;
+                fn = precise ? (const void*)kb_multiple_scattering<double, 4, H>
+                             : (const void*)kb_multiple_scattering<float, 4, H>;
             break;
     }
     int per_cu = 0, dev = 0, cus = 0;

@@ -146,6 +146,15 @@ fbk::DevParams make_dev_params(const fb_parameters& p) {
             d.prof[k][l].linear_term = src[k]->layers[l].linear_term;
             d.prof[k][l].constant_term = src[k]->layers[l].constant_term;
         }
+    // See MsCoord (precompute.hip).
+    const double B = d.bottom, T = d.top, H = std::sqrt(T * T - B * B);
+    const double range = H - (T - B), inv_a = range / (-2.0 * d.mu_s_min * B);
+    const double dm = (T - B) / range, h = H / range, top = double(d.s_mus - 1);
+    d.ms.c = float(B / H);
+    d.ms.c2 = float(B / H * (B / H));
+    d.ms.p0 = float((1.0 + dm * inv_a) / h * top);
+    d.ms.p1 = float(-inv_a * top);
+    d.ms.q0 = float((1.0 - dm) / h);
     return d;
 }
 

@@ -213,7 +213,8 @@ typedef struct fb_tuning {
     uint32_t xcd_remap; /* bit p set (p = FB_PASS_SINGLE_SCATTERING,
                            FB_PASS_SCATTERING_DENSITY or
                            FB_PASS_MULTIPLE_SCATTERING): that pass gives each
-                           of the 8 XCDs a contiguous share of its blocks */
+                           of the 8 XCDs a contiguous share of its blocks
+                           (untuned classes: multiple scattering only) */
     float best_ms[6]; /* fb_builder_autotune: measured ms per launch of each
                          chosen shape, in field order; 0 otherwise */
 } fb_tuning;
