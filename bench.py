@@ -10,7 +10,7 @@ loop (fb_server_submit_precomputes; continuous batching, at most 64
 precomputes in flight, 200 GB HBM budget, one precompute stream) and
 drained.  `value`
 is LUT sets per second over the timed steps and `latency_ms` the p50 / p99
-of the requests' submission-to-completion times.  Parameters are 272-byte
+of the requests' submission-to-completion times.  Parameters are 252-byte
 host structs; the LUTs stay resident in HBM, no host transfer is timed.
 
 Prints ONE JSON line.  Extra fields: the same set as one batch and through

@@ -22,7 +22,7 @@ CEILINGS_SOURCES = ["ceilings.hip"]
 
 ARCH = os.environ.get("FB_OFFLOAD_ARCH", "gfx950")
 
-SOURCES = ["precompute.hip", "render.hip", "runtime.hip", "batch.hip", "server.hip",
+SOURCES = ["density_f64.hip", "density_f32.hip", "precompute.hip", "render.hip", "runtime.hip", "batch.hip", "server.hip",
            "tune.hip", "noalloc.hip", "lutio.hip", "interop.hip"]
 
 COMMON = [

@@ -108,31 +108,11 @@ constexpr int kSsTexelsPerThread = 4;
 // texel would leave most of the device idle, each thread walking all 512
 // directions in sequence.
 constexpr size_t kDenSplitTexels = 65536;
-// Density texels per thread: 2 when the LUT set is not theta-split, NU is
-// even and an (r, mu_s) tile holds at least kDenPairMinTexels texels — the
-// thread then takes texels (mu, nu index k) and (mu, NU-1-k), which share
-// nu2 = omega.omega_i and the phase weight of every direction pair (computed
-// once for both), and a block's profile build serves twice the texels.
-constexpr int kDenPairMinTexels = 512;
-// Blocks per CU the density kernels are compiled for.  One texel per thread:
-// 4 (8 blocks, 64 VGPRs, spill: 0.066 instead of 0.041 ms per order >= 3
-// launch of a half-resolution set, whose blocks do not fill the chip).  Two:
-// 6 at order >= 3 (5: 2.69 instead of 2.60 ms at double), 5 at order 2 (6:
-// 5.30 instead of 5.23 ms).
-__host__ __device__ constexpr int den_occupancy(int tpx, bool single) {
-    return tpx == 1 ? 4 : (single ? 5 : 6);
-}
 // Whether the density pass runs the outer texels (nu index 0 and NU-1) on
 // their shortcut: precision mode.  FP32 mode follows the reference's
 // binary32 omega_s, which is off the meridian plane by its rounding, lookup
 // by lookup (with the shortcut one texel in 10^5 is 1e-4 from it).
 __host__ __device__ inline bool den_outer(const DevParams& P) { return P.flags & 1; }
-__host__ __device__ inline int den_tpx(const DevParams& P) {
-    return (P.den_split == 1 && (P.s_nu > 2 || !den_outer(P)) && P.s_nu % 2 == 0 &&
-            P.s_mu * P.s_nu >= kDenPairMinTexels)
-               ? 2
-               : 1;
-}
 // Row stride of the density kernel's table of outer incident radiance: 16
 // entries and one pad, so that the lanes of a theta-split group, each on its
 // own row, read from different banks.
@@ -147,11 +127,41 @@ struct DenLayout {
     __host__ __device__ DenLayout(const DevParams& P, int tpx) {
         const int split = tpx > 1 ? 1 : P.den_split;
         first = den_outer(P) ? 1 : 0;
-        groups = P.s_mu * (P.s_nu - 2 * first) / tpx;
+        groups = P.s_mu * ((P.s_nu - 2 * first) / tpx);
         inner = (groups * split + 63) / 64 * 64;
         total = inner + first * P.s_mu * split;
     }
 };
+// Density texels per thread.  The texels of one mu share nu2 = omega.omega_i
+// and the phase weight of every direction pair (13 of a lone texel's 34
+// instruction slots per pair), so a thread takes as many as divide the inner
+// nu indices evenly: 7, 6, 4 or 2, while the set's tiles fill at least
+// kDenMinWaves wavefronts (4 per SIMD; below that, occupancy is worth more
+// than the shared work).  Order >= 3 and order 2, ms per launch: double (14
+// inner) 7: 2.22 / 4.70, 4: 2.36 / 4.99 (2 of 16 places idle), 2: 2.42 / 5.11;
+// default (6 inner) 6: 0.168 / 0.325, 2: 0.174 / 0.348; default in FP32 mode
+// (8) 4: 0.181 / 0.385, 2: 0.189 / 0.408; 27x64x26x18 (16 inner, 3,510 waves
+// at 4) 4: 0.221 / 0.470, 2: 0.142 / 0.305.  A texel's own operations and
+// their order do not depend on it.
+constexpr int kDenMinWaves = 4096;
+constexpr int kDenPairMinTexels = 512;  // tiles of fewer texels keep one per thread
+__host__ __device__ inline int den_tpx(const DevParams& P) {
+    const int inner = P.s_nu - (den_outer(P) ? 2 : 0);
+    if (P.den_split != 1 || inner < 2) return 1;
+    const int tiles = P.s_mus * P.s_r;
+    for (int t = 7; t >= 4; --t)
+        if (t != 5 && inner % t == 0 && tiles * ((DenLayout(P, t).total + 63) / 64) >= kDenMinWaves)
+            return t;
+    return inner % 2 == 0 && P.s_mu * P.s_nu >= kDenPairMinTexels ? 2 : 1;
+}
+// Blocks of 256 threads per CU the density kernels are compiled for.  One
+// texel per thread: 4 (8 blocks, 64 VGPRs, spill: 0.066 instead of 0.041 ms
+// per order >= 3 launch of a half-resolution set, whose blocks do not fill
+// the chip).  Two: 7 at order >= 3, 5 at order 2 (at double 2.54 ms, 6 2.54,
+// 8 2.60; order 2 with 6 5.30 instead of 5.23).
+__host__ __device__ constexpr int den_occupancy(int tpx, bool single) {
+    return tpx == 2 ? (single ? 5 : 7) : tpx == 7 ? 3 : 4;
+}
 constexpr int kSsMaxStagedMu = 2048;
 // Multiple scattering over rows of at most kMsChunkMaxW texels (small LUT
 // sets, whose launches are a few hundred one-wavefront blocks, each walking
@@ -256,6 +266,19 @@ hipError_t launch_geometry(const DevParams& P, const float4* T, const float4* OD
 hipError_t launch_single_scattering(const DevParams& P, const float4* T, const float4* SR,
                                     float4* dR, float4* dM, float4* S, const Tuning& tu,
                                     hipStream_t s);
+// The scattering density kernels of geometry type G (one translation unit
+// each, density_f32.hip and density_f64.hip).
+template <typename G>
+struct DensityLaunch {
+    static hipError_t upload();
+    static hipError_t plain(const DevParams& P, int order, const float4* DG, const float4* dR,
+                            const float4* dM, const float4* dMS, const float4* dE, float4* J,
+                            unsigned threads, unsigned remap, hipStream_t s);
+    static void batch(bool single, bool f16, unsigned tpx, const DevParams* Ps, const LutPtrs* L,
+                      const uint32_t* tiles, unsigned ntiles, dim3 grid, dim3 block, size_t lds,
+                      hipStream_t s);
+    static const void* batch_kernel(bool single, bool f16, unsigned tpx);
+};
 hipError_t launch_scattering_density(const DevParams& P, int order, const float4* DG,
                                      const float4* dR, const float4* dM, const float4* dMS,
                                      const float4* dE, float4* J, const Tuning& tu,

@@ -4,8 +4,8 @@ the oracle's pass:
 
   * nu extents with only outer texels (2), one inner slice (3), and an even
     and an odd number of slices;
-  * theta-split sets (under 65,536 texels), one texel per thread, and two
-    texels per thread, none of them filling its wavefronts evenly;
+  * theta-split sets (under 65,536 texels), and one, two, four, six and
+    seven texels per thread, some not filling their wavefronts evenly;
   * an Earth-like planet (most ground rows meet no knot of the irradiance
     LUT) and a small one with a thick atmosphere under a fine irradiance LUT
     (rows of one knot and of many).
@@ -37,6 +37,12 @@ SIZES = {
                     scattering_nu_size=5),
     "pair_nu6": dict(scattering_r_size=8, scattering_mu_size=128, scattering_mu_s_size=11,
                      scattering_nu_size=6),
+    "four_nu6": dict(scattering_r_size=32, scattering_mu_size=72, scattering_mu_s_size=43,
+                     scattering_nu_size=6),
+    "six_nu8": dict(scattering_r_size=32, scattering_mu_size=72, scattering_mu_s_size=43,
+                    scattering_nu_size=8),
+    "seven_nu9": dict(scattering_r_size=32, scattering_mu_size=72, scattering_mu_s_size=43,
+                      scattering_nu_size=9),
 }
 PLANETS = {
     "earth": {},
