@@ -472,48 +472,4 @@ __device__ __forceinline__ TexelCoord<G> scattering_texel_coord(const DevParams&
     return c;
 }
 
-// Trilinear sample of a packed scattering LUT at texel coordinate
-// (x within [0, W), u_mu, u_r) — the (y, z) taps are shared by the caller.
-struct Taps3 {
-    Taps y, z;
-};
-
-// scattering.h:139-155: GetScattering on one texture, nu lerped manually
-// between two trilinear samples at slices floor(u_nu*(NU-1)) and +1.  H: the
-// texture is binary16 (FB_FLAG_F16_STORAGE).
-template <typename G, bool H>
-__device__ __forceinline__ float4 get_scattering_tex(const DevParams& P,
-                                                     const float4* __restrict__ tex, G r, G mu,
-                                                     G mu_s, G nu, bool ground) {
-    G u_r = scattering_u_r<G>(P, r);
-    G u_mu = scattering_u_mu<G>(P, r, mu, ground);
-    G u_mu_s = scattering_u_mu_s<G>(P, mu_s);
-    G u_nu = (nu + G(1)) / G(2);
-    G tex_coord_x = u_nu * G(P.s_nu - 1);
-    G tex_x = floor(tex_coord_x);
-    float lerp = float(tex_coord_x - tex_x);
-    G x0 = (tex_x + u_mu_s) / G(P.s_nu);
-    G x1 = (tex_x + G(1) + u_mu_s) / G(P.s_nu);
-    int W = P.s_nu * P.s_mus;
-    Taps ty = linear_taps<G>(u_mu, P.s_mu), tz = linear_taps<G>(u_r, P.s_r);
-    Taps tx0 = linear_taps<G>(x0, W), tx1 = linear_taps<G>(x1, W);
-    const size_t p00 = (size_t(tz.i0) * P.s_mu + ty.i0) * W;
-    const size_t p01 = (size_t(tz.i0) * P.s_mu + ty.i1) * W;
-    const size_t p10 = (size_t(tz.i1) * P.s_mu + ty.i0) * W;
-    const size_t p11 = (size_t(tz.i1) * P.s_mu + ty.i1) * W;
-    auto at = [&](size_t row, int x) { return ld_tex(tex, row + x, H); };
-    float4 a0 = lerp4(lerp4(lerp4(at(p00, tx0.i0), at(p00, tx0.i1), tx0.w),
-                            lerp4(at(p01, tx0.i0), at(p01, tx0.i1), tx0.w), ty.w),
-                      lerp4(lerp4(at(p10, tx0.i0), at(p10, tx0.i1), tx0.w),
-                            lerp4(at(p11, tx0.i0), at(p11, tx0.i1), tx0.w), ty.w),
-                      tz.w);
-    float4 a1 = lerp4(lerp4(lerp4(at(p00, tx1.i0), at(p00, tx1.i1), tx1.w),
-                            lerp4(at(p01, tx1.i0), at(p01, tx1.i1), tx1.w), ty.w),
-                      lerp4(lerp4(at(p10, tx1.i0), at(p10, tx1.i1), tx1.w),
-                            lerp4(at(p11, tx1.i0), at(p11, tx1.i1), tx1.w), ty.w),
-                      tz.w);
-    return make_float4(a0.x * (1.0f - lerp) + a1.x * lerp, a0.y * (1.0f - lerp) + a1.y * lerp,
-                       a0.z * (1.0f - lerp) + a1.z * lerp, a0.w * (1.0f - lerp) + a1.w * lerp);
-}
-
 }  // namespace fbk

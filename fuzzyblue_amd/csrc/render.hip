@@ -14,25 +14,247 @@ __device__ __forceinline__ float dot3(float3 a, float3 b) {
     return a.x * b.x + a.y * b.y + a.z * b.z;
 }
 
-// render_sky.h:9-19
-__device__ __forceinline__ float3 extrapolated_single_mie(const DevParams& P, float4 s) {
-    if (s.x <= 0.0f) return make_float3(0.0f, 0.0f, 0.0f);
-    float k = P.rayleigh_scattering[0] / P.mie_scattering[0];
-    return make_float3(s.x * s.w / s.x * k * (P.mie_scattering[0] / P.rayleigh_scattering[0]),
-                       s.y * s.w / s.x * k * (P.mie_scattering[1] / P.rayleigh_scattering[1]),
-                       s.z * s.w / s.x * k * (P.mie_scattering[2] / P.rayleigh_scattering[2]));
+// a / b correctly rounded, given y = 1/b correctly rounded and b normal: q =
+// a*y, then Markstein's correction q + (a - b*q)*y with the residual exact
+// in an FMA (P. Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", IBM J. Res. Dev. 34(1), 1990) -- three
+// instructions in place of an IEEE division's ten, the same bits.  The
+// residual is a multiple of about 2^(e_a - 46): for numerators below 2^-80
+// (other than 0) it can be subnormal or not representable, and a wavefront
+// with such a lane takes the division (a wave-uniform branch; the empty asm
+// statement keeps the compiler from evaluating the division unconditionally
+// and selecting).
+__device__ __forceinline__ float div_rn(float a, float b, float y) {
+    const float q = a * y;
+    float d = fmaf(fmaf(-q, b, a), y, q);
+    if (__builtin_amdgcn_ballot_w64(a != 0.0f && fabsf(a) < 0x1p-80f)) {
+        asm volatile("");
+        d = a / b;
+    }
+    return d;
 }
 
-// render_sky.h:21-43 (GLSL mix of the two nu slices).  H: the scattering LUT
-// is binary16 (FB_FLAG_F16_STORAGE); every function and kernel below that
-// reads it takes the same parameter.
+// a / b for normal b of ordinary size: a reciprocal refined once, then
+// Markstein's correction -- 9 instruction slots, the compiler's IEEE division
+// about 16.  The refined reciprocal is within an ulp, so the quotient is the
+// IEEE one but for about one pair in 2^23, off by an ulp.
+__device__ __forceinline__ float div_nr(float a, float b) {
+    float y = __builtin_amdgcn_rcpf(b);
+    y = fmaf(fmaf(-b, y, 1.0f), y, y);
+    const float q = a * y;
+    return fmaf(fmaf(-b, q, a), y, q);
+}
+// The same where a wavefront's operands are of ordinary size, else a / b.
+__device__ __forceinline__ float div_any(float a, float b) {
+    float d = div_nr(a, b);
+    if (__builtin_amdgcn_ballot_w64(!(fabsf(b) > 0x1p-100f && fabsf(b) < 0x1p100f &&
+                                      fabsf(a) < 0x1p100f))) {
+        asm volatile("");
+        d = a / b;
+    }
+    return d;
+}
+// sqrt(max(x, 0)) from the hardware's reciprocal square root by two coupled
+// Newton steps, the second with the exact residual: the IEEE root but for
+// rare arguments (an ulp), 13 slots instead of about 20.
+__device__ __forceinline__ float sqrt_nr(float x) {
+    x = fmaxf(x, 0.0f);
+    const float y = __builtin_amdgcn_rsqf(x);
+    float g = x * y, h = 0.5f * y;
+    const float r = fmaf(-h, g, 0.5f);
+    g = fmaf(g, r, g);
+    h = fmaf(h, r, h);
+    g = fmaf(fmaf(-g, g, x), h, g);
+    return x < 0x1p-60f ? __builtin_amdgcn_sqrtf(x) : g;
+}
+
+// The constants of the lookups that depend on the atmosphere and the LUT
+// extents only, evaluated once on the host by the reference's expressions in
+// the same binary32 operations (neither compiler pass fuses or reorders
+// them), so a lookup's coordinates keep their bits.
+struct SkyLut {
+    float bottom, top, b2, t2;          // radii and their squares
+    float h, h_inv, h2;                 // sqrt(top^2 - bottom^2), 1 / h, h * h
+    float t_u0, t_u1, t_v0, t_v1;       // tex_from_unit(x, n) = u0 + x * u1: t_mu, t_r
+    float r0, r1, m0, m1, s0, s1;       // ... s_r, s_mu / 2, s_mus
+    float ms_dmin, ms_den, ms_inv, ms_a, ms_a_inv;  // scattering.h:48-56
+    float nu_den, nu_inv;               // s_nu, 1 / s_nu
+    float mie_k, mie[3];                // rayleigh.r / mie.r, mie / rayleigh
+    float pm_k, pm_g1, pm_g2;           // phase_mie: k, 1 + g^2, 2g
+    int t_mu, t_r, s_r, s_mu, s_mus, s_nu;
+};
+__host__ __device__ inline SkyLut sky_lut(const DevParams& P) {
+    SkyLut L;
+    const float b = P.bottom, t = P.top;
+    L.bottom = b;
+    L.top = t;
+    L.b2 = b * b;
+    L.t2 = t * t;
+    L.h = sqrtf(t * t - b * b);
+    L.h_inv = 1.0f / L.h;
+    L.h2 = L.h * L.h;
+    L.t_u0 = 0.5f / float(P.t_mu);
+    L.t_u1 = 1.0f - 1.0f / float(P.t_mu);
+    L.t_v0 = 0.5f / float(P.t_r);
+    L.t_v1 = 1.0f - 1.0f / float(P.t_r);
+    L.r0 = 0.5f / float(P.s_r);
+    L.r1 = 1.0f - 1.0f / float(P.s_r);
+    const int hm = P.s_mu / 2;
+    L.m0 = 0.5f / float(hm);
+    L.m1 = 1.0f - 1.0f / float(hm);
+    L.s0 = 0.5f / float(P.s_mus);
+    L.s1 = 1.0f - 1.0f / float(P.s_mus);
+    L.ms_dmin = t - b;
+    L.ms_den = L.h - L.ms_dmin;
+    L.ms_inv = 1.0f / L.ms_den;
+    L.ms_a = -2.0f * P.mu_s_min * b / L.ms_den;
+    L.ms_a_inv = 1.0f / L.ms_a;
+    L.nu_den = float(P.s_nu);
+    L.nu_inv = 1.0f / L.nu_den;
+    // render_sky.h:9-19
+    L.mie_k = P.rayleigh_scattering[0] / P.mie_scattering[0];
+    for (int i = 0; i < 3; ++i) L.mie[i] = P.mie_scattering[i] / P.rayleigh_scattering[i];
+    // util.h:31-34
+    const float g = P.g;
+    L.pm_k = 3.0f / (8.0f * kPi) * (1.0f - g * g) / (2.0f + g * g);
+    L.pm_g1 = 1.0f + g * g;
+    L.pm_g2 = 2.0f * g;
+    L.t_mu = P.t_mu;
+    L.t_r = P.t_r;
+    L.s_r = P.s_r;
+    L.s_mu = P.s_mu;
+    L.s_mus = P.s_mus;
+    L.s_nu = P.s_nu;
+    return L;
+}
+
+// distance_to_top (params.h:105-110) and transmittance.h:7-33.
+__device__ __forceinline__ float lut_d_top(const SkyLut& L, float r, float mu) {
+    return fmaxf(-r * mu + sqrt_nr(r * r * (mu * mu - 1.0f) + L.t2), 0.0f);
+}
+__device__ __forceinline__ float3 lut_transmittance(const SkyLut& L,
+                                                    const float4* __restrict__ T, float r,
+                                                    float mu) {
+    const float rho = sqrt_nr(r * r - L.b2);
+    const float d_min = L.top - r, d_max = rho + L.h;
+    const float x_mu = div_nr(lut_d_top(L, r, mu) - d_min, d_max - d_min);
+    const float u = L.t_u0 + x_mu * L.t_u1;
+    const float v = L.t_v0 + div_rn(rho, L.h, L.h_inv) * L.t_v1;
+    const float4 t = sample2d<float>(T, L.t_mu, L.t_r, u, v);
+    return make_float3(t.x, t.y, t.z);
+}
+// min(n / q, 1) per channel (transmittance.h:53-60).
+__device__ __forceinline__ float3 lut_ratio(float3 n, float3 q) {
+    return make_float3(fminf(div_any(n.x, q.x), 1.0f), fminf(div_any(n.y, q.y), 1.0f),
+                       fminf(div_any(n.z, q.z), 1.0f));
+}
+// transmittance.h:35-61
+__device__ __forceinline__ float3 lut_segment(const SkyLut& L, const float4* __restrict__ T,
+                                              float r, float mu, float d, bool ground) {
+    const float r_d = fminf(fmaxf(sqrtf(d * d + 2.0f * r * mu * d + r * r), L.bottom), L.top);
+    const float mu_d = clamp_cosine<float>((r * mu + d) / r_d);
+    const float3 far = lut_transmittance(L, T, r_d, ground ? -mu_d : mu_d);
+    const float3 near = lut_transmittance(L, T, r, ground ? -mu : mu);
+    const float3 n = ground ? far : near, q = ground ? near : far;
+    return lut_ratio(n, q);
+}
+// scattering.h:28-46: the mu coordinate.
+__device__ __forceinline__ float lut_u_mu(const SkyLut& L, float r, float rho, float mu,
+                                          bool ground) {
+    const float r_mu = r * mu;
+    const float disc = r_mu * r_mu - r * r + L.b2;
+    // One square root and one division for both kinds of ray.
+    const float root = sqrt_nr(ground ? disc : disc + L.h2);
+    const float d = ground ? -r_mu - root : -r_mu + root;
+    const float d_min = ground ? r - L.bottom : L.top - r;
+    const float d_max = ground ? rho : rho + L.h;
+    const float x = ground && d_max == d_min ? 0.0f : div_nr(d - d_min, d_max - d_min);
+    const float u = 0.5f * (L.m0 + x * L.m1);
+    return ground ? 0.5f - u : 0.5f + u;
+}
+// Two neighbouring texels of a row, taps i0 and i1 of linear_taps (i0 + 1 =
+// i1, or both the same edge texel).  Binary16 texels take one 16-byte load.
 template <bool H>
-__device__ __forceinline__ float4 combined_scattering(const DevParams& P,
+__device__ __forceinline__ float4 row_lerp(const float4* __restrict__ tex, size_t row, int w,
+                                           const Taps& t) {
+    if constexpr (H) {
+        typedef _Float16 Half8 __attribute__((ext_vector_type(8), aligned(8)));
+        const int b = min(t.i0, w - 2);
+        const Half8 v =
+            *reinterpret_cast<const Half8*>(reinterpret_cast<const Half4*>(tex) + row + b);
+        const float4 lo = widen4(__builtin_shufflevector(v, v, 0, 1, 2, 3)),
+                     hi = widen4(__builtin_shufflevector(v, v, 4, 5, 6, 7));
+        const bool a = t.i0 != b, c = t.i1 != b;
+        return lerp4(make_float4(a ? hi.x : lo.x, a ? hi.y : lo.y, a ? hi.z : lo.z,
+                                 a ? hi.w : lo.w),
+                     make_float4(c ? hi.x : lo.x, c ? hi.y : lo.y, c ? hi.z : lo.z,
+                                 c ? hi.w : lo.w),
+                     t.w);
+    } else {
+        return lerp4(ldg4(tex + row + t.i0), ldg4(tex + row + t.i1), t.w);
+    }
+}
+// scattering.h:139-155: GetScattering on one texture, nu lerped manually
+// between two trilinear samples at slices floor(u_nu*(NU-1)) and +1.  H: the
+// texture is binary16 (FB_FLAG_F16_STORAGE); every function and kernel below
+// that reads it takes the same parameter.
+template <bool H>
+__device__ __forceinline__ float4 lut_scattering(const SkyLut& L, const float4* __restrict__ tex,
+                                                 float r, float mu, float mu_s, float nu,
+                                                 bool ground) {
+    const float rho = sqrt_nr(r * r - L.b2);
+    const float u_r = L.r0 + div_rn(rho, L.h, L.h_inv) * L.r1;
+    const float u_mu = lut_u_mu(L, r, rho, mu, ground);
+    const float d =
+        fmaxf(-L.bottom * mu_s + sqrt_nr(L.b2 * (mu_s * mu_s - 1.0f) + L.t2), 0.0f);
+    const float a = div_rn(d - L.ms_dmin, L.ms_den, L.ms_inv);
+    const float u_mu_s =
+        L.s0 + div_nr(fmaxf(1.0f - div_rn(a, L.ms_a, L.ms_a_inv), 0.0f), 1.0f + a) * L.s1;
+    const float tex_coord_x = (nu + 1.0f) / 2.0f * float(L.s_nu - 1);
+    const float tex_x = floorf(tex_coord_x);
+    const float lerp = tex_coord_x - tex_x;
+    const int W = L.s_nu * L.s_mus;
+    const Taps ty = linear_taps<float>(u_mu, L.s_mu), tz = linear_taps<float>(u_r, L.s_r);
+    const Taps tx0 = linear_taps<float>(div_rn(tex_x + u_mu_s, L.nu_den, L.nu_inv), W);
+    const Taps tx1 = linear_taps<float>(div_rn(tex_x + 1.0f + u_mu_s, L.nu_den, L.nu_inv), W);
+    const size_t p00 = (size_t(tz.i0) * L.s_mu + ty.i0) * W;
+    const size_t p01 = (size_t(tz.i0) * L.s_mu + ty.i1) * W;
+    const size_t p10 = (size_t(tz.i1) * L.s_mu + ty.i0) * W;
+    const size_t p11 = (size_t(tz.i1) * L.s_mu + ty.i1) * W;
+    const float4 a0 = lerp4(
+        lerp4(row_lerp<H>(tex, p00, W, tx0), row_lerp<H>(tex, p01, W, tx0), ty.w),
+        lerp4(row_lerp<H>(tex, p10, W, tx0), row_lerp<H>(tex, p11, W, tx0), ty.w), tz.w);
+    const float4 a1 = lerp4(
+        lerp4(row_lerp<H>(tex, p00, W, tx1), row_lerp<H>(tex, p01, W, tx1), ty.w),
+        lerp4(row_lerp<H>(tex, p10, W, tx1), row_lerp<H>(tex, p11, W, tx1), ty.w), tz.w);
+    return make_float4(a0.x * (1.0f - lerp) + a1.x * lerp, a0.y * (1.0f - lerp) + a1.y * lerp,
+                       a0.z * (1.0f - lerp) + a1.z * lerp, a0.w * (1.0f - lerp) + a1.w * lerp);
+}
+
+// render_sky.h:9-19, the red channel (s.x * s.w / s.x * k * ratio) and all.
+__device__ __forceinline__ float single_mie_red(const SkyLut& L, float4 s) {
+    return s.x <= 0.0f ? 0.0f : div_any(s.x * s.w, s.x) * L.mie_k * L.mie[0];
+}
+__device__ __forceinline__ float3 extrapolated_single_mie(const SkyLut& L, float4 s) {
+    if (s.x <= 0.0f) return make_float3(0.0f, 0.0f, 0.0f);
+    const float q = div_any(s.w, s.x);
+    return make_float3(s.x * q * L.mie_k * L.mie[0], s.y * q * L.mie_k * L.mie[1],
+                       s.z * q * L.mie_k * L.mie[2]);
+}
+// util.h:31-34, x^-1.5 by the hardware's reciprocal square root (a few ulp).
+__device__ __forceinline__ float lut_phase_mie(const SkyLut& L, float nu) {
+    const float y = __builtin_amdgcn_rsqf(L.pm_g1 - L.pm_g2 * nu);
+    return L.pm_k * (1.0f + nu * nu) * (y * y * y);
+}
+
+// render_sky.h:21-43 (GLSL mix of the two nu slices).
+template <bool H>
+__device__ __forceinline__ float4 combined_scattering(const DevParams& P, const SkyLut& L,
                                                       const float4* __restrict__ S, float r,
                                                       float mu, float mu_s, float nu, bool ground,
                                                       float3& mie) {
-    float4 c = get_scattering_tex<float, H>(P, S, r, mu, mu_s, nu, ground);
-    mie = extrapolated_single_mie(P, c);
+    float4 c = lut_scattering<H>(L, S, r, mu, mu_s, nu, ground);
+    mie = extrapolated_single_mie(L, c);
     return c;
 }
 
@@ -40,7 +262,7 @@ __device__ __forceinline__ float4 combined_scattering(const DevParams& P,
 // keeps commented out (render_sky.h:81-106) for shadow_length > 0; a
 // shadow_length of 0 is the reference's path.
 template <bool H, bool SHADOW = false>
-__device__ void sky_radiance(const DevParams& P, const float4* __restrict__ T,
+__device__ void sky_radiance(const DevParams& P, const SkyLut& L, const float4* __restrict__ T,
                              const float4* __restrict__ S, float3 camera, float3 view,
                              float3 sun, float3& rad, float3& trans,
                              float shadow_length = 0.0f) {
@@ -61,11 +283,11 @@ __device__ void sky_radiance(const DevParams& P, const float4* __restrict__ T,
     float mu_s = dot3(camera, sun) / r;
     float nu = dot3(view, sun);
     bool ground = ray_intersects_ground<float>(P, r, mu);
-    trans = ground ? make_float3(0.0f, 0.0f, 0.0f) : transmittance_to_top<float>(P, T, r, mu);
+    trans = ground ? make_float3(0.0f, 0.0f, 0.0f) : lut_transmittance(L, T, r, mu);
     float3 mie;
     float4 sc;
     if (!SHADOW || shadow_length == 0.0f) {
-        sc = combined_scattering<H>(P, S, r, mu, mu_s, nu, ground, mie);
+        sc = combined_scattering<H>(P, L, S, r, mu, mu_s, nu, ground, mie);
     } else {
         // Eq. (18): the scattering seen from x + l v, attenuated by
         // T(x, x + l v) (render_sky.h:86-105).
@@ -73,20 +295,20 @@ __device__ void sky_radiance(const DevParams& P, const float4* __restrict__ T,
         const float r_p = clamp_radius<float>(P, sqrtf(d * d + 2.0f * r * mu * d + r * r));
         const float mu_p = (r * mu + d) / r_p;
         const float mu_s_p = (r * mu_s + d * nu) / r_p;
-        sc = combined_scattering<H>(P, S, r_p, mu_p, mu_s_p, nu, ground, mie);
-        const float3 st = get_transmittance<float>(P, T, r, mu, shadow_length, ground);
+        sc = combined_scattering<H>(P, L, S, r_p, mu_p, mu_s_p, nu, ground, mie);
+        const float3 st = lut_segment(L, T, r, mu, shadow_length, ground);
         sc = make_float4(sc.x * st.x, sc.y * st.y, sc.z * st.z, sc.w);
         mie = make_float3(mie.x * st.x, mie.y * st.y, mie.z * st.z);
     }
-    float pr = phase_rayleigh(nu), pm = phase_mie(P.g, nu);
+    float pr = phase_rayleigh(nu), pm = lut_phase_mie(L, nu);
     rad = make_float3(sc.x * pr + mie.x * pm, sc.y * pr + mie.y * pm, sc.z * pr + mie.z * pm);
 }
 
 // render_sky.h:111-191, with the commented-out light-shaft term
 // (:158-160, :172-177) when SHADOW and shadow_length > 0.
 template <bool H, bool SHADOW = false>
-__device__ void sky_radiance_to_point(const DevParams& P, const float4* __restrict__ T,
-                                      const float4* __restrict__ S, float3 camera, float3 view,
+__device__ void sky_radiance_to_point(const DevParams& P, const SkyLut& L,
+                                      const float4* __restrict__ T, const float4* __restrict__ S, float3 camera, float3 view,
                                       float3 point, float3 sun, float3& rad, float3& trans,
                                       float shadow_length = 0.0f) {
     float r = sqrtf(dot3(camera, camera));
@@ -108,30 +330,30 @@ __device__ void sky_radiance_to_point(const DevParams& P, const float4* __restri
     float3 pc = make_float3(point.x - camera.x, point.y - camera.y, point.z - camera.z);
     float d = sqrtf(dot3(pc, pc));
     bool ground = ray_intersects_ground<float>(P, r, mu);
-    trans = get_transmittance<float>(P, T, r, mu, d, ground);
+    trans = lut_segment(L, T, r, mu, d, ground);
     float3 mie;
-    float4 sc = combined_scattering<H>(P, S, r, mu, mu_s, nu, ground, mie);
+    float4 sc = combined_scattering<H>(P, L, S, r, mu, mu_s, nu, ground, mie);
     if (!isinf(d)) {
         // Eq. (17): the second lookup at d - l, attenuated by T(x, x_{d-l}).
         float3 st = trans;
         if (SHADOW && shadow_length > 0.0f) {
             d = fmaxf(d - shadow_length, 0.0f);
-            st = get_transmittance<float>(P, T, r, mu, d, ground);
+            st = lut_segment(L, T, r, mu, d, ground);
         }
         float r_p = clamp_radius<float>(P, sqrtf(d * d + 2.0f * r * mu * d + r * r));
         float mu_p = (r * mu + d) / r_p;
         float mu_s_p = (r * mu_s + d * nu) / r_p;
         float3 mie_p;
-        float4 sc_p = combined_scattering<H>(P, S, r_p, mu_p, mu_s_p, nu, ground, mie_p);
+        float4 sc_p = combined_scattering<H>(P, L, S, r_p, mu_p, mu_s_p, nu, ground, mie_p);
         sc.x = sc.x - st.x * sc_p.x;
         sc.y = sc.y - st.y * sc_p.y;
         sc.z = sc.z - st.z * sc_p.z;
         float mr = mie.x - st.x * mie_p.x;
-        mie = extrapolated_single_mie(P, make_float4(sc.x, sc.y, sc.z, mr));
+        mie = extrapolated_single_mie(L, make_float4(sc.x, sc.y, sc.z, mr));
         float h = smoothstep_g<float>(0.0f, 0.01f, mu_s);
         mie = make_float3(mie.x * h, mie.y * h, mie.z * h);
     }
-    float pr = phase_rayleigh(nu), pm = phase_mie(P.g, nu);
+    float pr = phase_rayleigh(nu), pm = lut_phase_mie(L, nu);
     rad = make_float3(sc.x * pr + mie.x * pm, sc.y * pr + mie.y * pm, sc.z * pr + mie.z * pm);
 }
 
@@ -176,26 +398,6 @@ __device__ void build_sky_slice(const DevParams& P, const float4* __restrict__ T
         trow[m] = lerp4(ldg4(T + tv.i0 * TMU + m), ldg4(T + tv.i1 * TMU + m), tv.w);
 }
 
-// a / b correctly rounded, given y = 1/b correctly rounded and b normal: q =
-// a*y, then Markstein's correction q + (a - b*q)*y with the residual exact
-// in an FMA (P. Markstein, "Computation of elementary functions on the IBM
-// RISC System/6000 processor", IBM J. Res. Dev. 34(1), 1990) -- three
-// instructions in place of an IEEE division's ten, the same bits.  The
-// residual is a multiple of about 2^(e_a - 46): for numerators below 2^-80
-// (other than 0) it can be subnormal or not representable, and a wavefront
-// with such a lane takes the division (a wave-uniform branch; the empty asm
-// statement keeps the compiler from evaluating the division unconditionally
-// and selecting).
-__device__ __forceinline__ float div_rn(float a, float b, float y) {
-    const float q = a * y;
-    float d = fmaf(fmaf(-q, b, a), y, q);
-    if (__builtin_amdgcn_ballot_w64(a != 0.0f && fabsf(a) < 0x1p-80f)) {
-        asm volatile("");
-        d = a / b;
-    }
-    return d;
-}
-
 // The per-frame terms of sky_radiance_slice: everything that depends on
 // the camera's r and the atmosphere only, computed once per block.
 struct SliceConsts {
@@ -209,7 +411,7 @@ struct SliceConsts {
     float mie[3];                 // (rayleigh.r / mie.r) * (mie / rayleigh)
     float pm_k, pm_g1, pm_g2;     // phase_mie: k, 1 + g^2, 2g
 };
-__device__ inline SliceConsts slice_consts(const DevParams& P, float r) {
+__host__ __device__ inline SliceConsts slice_consts(const DevParams& P, float r) {
     SliceConsts c;
     const float b = P.bottom, t = P.top;
     c.r = r;
@@ -247,6 +449,48 @@ __device__ inline SliceConsts slice_consts(const DevParams& P, float r) {
     return c;
 }
 
+// transmittance.h:26-33 at the slice's r.
+__device__ __forceinline__ float3 slice_transmittance(const SliceConsts& C,
+                                                      const float4* __restrict__ trow, int t_mu,
+                                                      float mu) {
+    // distance_to_top (params.h:105-110), then transmittance.h:7-24's u
+    const float disc = C.rr * (mu * mu - 1.0f) + C.t2;
+    const float d = fmaxf(-C.r * mu + sqrt_nr(disc), 0.0f);
+    const float u = C.t_u0 + div_rn(d - C.t_dmin, C.t_den, C.t_inv) * C.t_u1;
+    const Taps tu = linear_taps<float>(u, t_mu);
+    const float4 t = lerp4(trow[tu.i0], trow[tu.i1], tu.w);
+    return make_float3(t.x, t.y, t.z);
+}
+// scattering.h:139-155 at the slice's r and mu_s.
+__device__ __forceinline__ float4 slice_scattering(const SliceConsts& C,
+                                                   const float4* __restrict__ slice, int NU,
+                                                   int MU, float mu, float nu, bool ground) {
+    // scattering.h:23-46
+    const float r_mu = C.r * mu;
+    const float disc = r_mu * r_mu - C.rr + C.b2;
+    float u_mu;
+    if (ground) {
+        const float d = -r_mu - sqrt_nr(disc);
+        const float x = C.g_den == 0.0f ? 0.0f : div_rn(d - C.g_dmin, C.g_den, C.g_inv);
+        u_mu = 0.5f - 0.5f * (C.m_u0 + x * C.m_u1);
+    } else {
+        const float d = -r_mu + sqrt_nr(disc + C.h2);
+        u_mu = 0.5f + 0.5f * (C.m_u0 + div_rn(d - C.s_dmin, C.s_den, C.s_inv) * C.m_u1);
+    }
+    const Taps ty = linear_taps<float>(u_mu, MU);
+    // nu of unit vectors can round just below -1 (anti-solar rays): clamped
+    // so the slice index stays >= 0.  The per-ray lookup's CLAMP_TO_EDGE
+    // then gives the same value up to a weight of the rounding's size.
+    const float tex_coord_x = (fminf(fmaxf(nu, -1.0f), 1.0f) + 1.0f) / 2.0f * float(NU - 1);
+    const float tex_x = floorf(tex_coord_x);
+    const float l = tex_coord_x - tex_x;
+    const int k0 = int(tex_x);
+    const float4 a0 = lerp4(slice[k0 * MU + ty.i0], slice[k0 * MU + ty.i1], ty.w);
+    const float4 a1 = lerp4(slice[(k0 + 1) * MU + ty.i0], slice[(k0 + 1) * MU + ty.i1], ty.w);
+    return make_float4(a0.x * (1.0f - l) + a1.x * l, a0.y * (1.0f - l) + a1.y * l,
+                       a0.z * (1.0f - l) + a1.z * l, a0.w * (1.0f - l) + a1.w * l);
+}
+
 // sky_radiance for a camera inside the atmosphere (so no move to the top
 // boundary), from the block's slice at the camera's r and mu_s.  Every
 // lookup coordinate is the reference's expression in the same binary32
@@ -263,46 +507,12 @@ __device__ void sky_radiance_slice(const DevParams& P, const SliceConsts& C,
                                    const float4* __restrict__ lds, float3 camera, float3 view,
                                    float3 sun, float3& rad, float3& trans) {
     const int NU = P.s_nu, MU = P.s_mu;
-    const float r = C.r;
-    const float mu = div_rn(dot3(camera, view), r, C.r_inv);
+    const float mu = div_rn(dot3(camera, view), C.r, C.r_inv);
     const float nu = dot3(view, sun);
-    const bool ground = ray_intersects_ground<float>(P, r, mu);
-    if (ground) {
-        trans = make_float3(0.0f, 0.0f, 0.0f);
-    } else {
-        // distance_to_top (params.h:105-110), then transmittance.h:7-24's u
-        const float disc = C.rr * (mu * mu - 1.0f) + C.t2;
-        const float d = fmaxf(-r * mu + sqrtf(fmaxf(disc, 0.0f)), 0.0f);
-        const float u = C.t_u0 + div_rn(d - C.t_dmin, C.t_den, C.t_inv) * C.t_u1;
-        const Taps tu = linear_taps<float>(u, P.t_mu);
-        const float4* trow = lds + (NU + 1) * MU;
-        const float4 t = lerp4(trow[tu.i0], trow[tu.i1], tu.w);
-        trans = make_float3(t.x, t.y, t.z);
-    }
-    // scattering.h:23-46
-    const float r_mu = r * mu;
-    const float disc = r_mu * r_mu - C.rr + C.b2;
-    float u_mu;
-    if (ground) {
-        const float d = -r_mu - sqrtf(fmaxf(disc, 0.0f));
-        const float x = C.g_den == 0.0f ? 0.0f : div_rn(d - C.g_dmin, C.g_den, C.g_inv);
-        u_mu = 0.5f - 0.5f * (C.m_u0 + x * C.m_u1);
-    } else {
-        const float d = -r_mu + sqrtf(fmaxf(disc + C.h2, 0.0f));
-        u_mu = 0.5f + 0.5f * (C.m_u0 + div_rn(d - C.s_dmin, C.s_den, C.s_inv) * C.m_u1);
-    }
-    const Taps ty = linear_taps<float>(u_mu, MU);
-    // nu of unit vectors can round just below -1 (anti-solar rays): clamped
-    // so the slice index stays >= 0.  The per-ray lookup's CLAMP_TO_EDGE
-    // then gives the same value up to a weight of the rounding's size.
-    const float tex_coord_x = (fminf(fmaxf(nu, -1.0f), 1.0f) + 1.0f) / 2.0f * float(NU - 1);
-    const float tex_x = floorf(tex_coord_x);
-    const float l = tex_coord_x - tex_x;
-    const int k0 = int(tex_x);
-    const float4 a0 = lerp4(lds[k0 * MU + ty.i0], lds[k0 * MU + ty.i1], ty.w);
-    const float4 a1 = lerp4(lds[(k0 + 1) * MU + ty.i0], lds[(k0 + 1) * MU + ty.i1], ty.w);
-    const float4 c = make_float4(a0.x * (1.0f - l) + a1.x * l, a0.y * (1.0f - l) + a1.y * l,
-                                 a0.z * (1.0f - l) + a1.z * l, a0.w * (1.0f - l) + a1.w * l);
+    const bool ground = ray_intersects_ground<float>(P, C.r, mu);
+    trans = ground ? make_float3(0.0f, 0.0f, 0.0f)
+                   : slice_transmittance(C, lds + (NU + 1) * MU, P.t_mu, mu);
+    const float4 c = slice_scattering(C, lds, NU, MU, mu, nu, ground);
     // render_sky.h:9-19
     float3 mie = make_float3(0.0f, 0.0f, 0.0f);
     if (c.x > 0.0f) {
@@ -315,6 +525,12 @@ __device__ void sky_radiance_slice(const DevParams& P, const SliceConsts& C,
     rad = make_float3(c.x * pr + mie.x * pm, c.y * pr + mie.y * pm, c.z * pr + mie.z * pm);
 }
 
+// Draws of fewer pixels look the LUTs up directly: the slice costs a launch
+// and a stream-ordered allocation.  us per draw, slice / direct: 640x360 23.9 /
+// 15.9, 1280x720 38.4 / 36.2, 1920x1080 62.9 / 69.4 (binary16 53.6 / 70.6),
+// 3840x2160 190 / 230.
+constexpr size_t kDrawSliceMinPixels = 1500000;
+
 struct DrawArgs {
     float ivp[4][4];  // [column][row]
     float cam[3];
@@ -323,32 +539,24 @@ struct DrawArgs {
 
 // render_sky.frag:24-35 for one pixel; fullscreen.vert:5-8 interpolates
 // screen_coords to ((px+0.5)/w, (py+0.5)/h) at pixel centres.
-template <bool H>
-__global__ __launch_bounds__(256) void k_render_sky(DevParams P, const float4* __restrict__ T,
-                                                    const float4* __restrict__ S, DrawArgs D,
-                                                    const float* __restrict__ depth, int w, int h,
-                                                    float4* __restrict__ color,
-                                                    float4* __restrict__ trans_out,
-                                                    int composite) {
-    int px = blockIdx.x * 16 + (threadIdx.x % 16);
-    int py = blockIdx.y * 16 + (threadIdx.x / 16);
-    if (px >= w || py >= h) return;
-    size_t idx = size_t(py) * w + px;
-    float sx = (float(px) + 0.5f) / float(w), sy = (float(py) + 0.5f) / float(h);
+__device__ __forceinline__ void unproject(const DrawArgs& D, int px, int py, int w, int h,
+                                          float dz, float3& view, float3& world) {
+    float sx = div_nr(float(px) + 0.5f, float(w)), sy = div_nr(float(py) + 0.5f, float(h));
     float n0 = 2.0f * sx - 1.0f, n1 = 2.0f * sy - 1.0f;
     float v[4];
     for (int row = 0; row < 4; ++row)
         v[row] = D.ivp[0][row] * n0 + D.ivp[1][row] * n1 + D.ivp[2][row] * 0.0f + D.ivp[3][row];
-    float len = sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    float3 view = make_float3(v[0] / len, v[1] / len, v[2] / len);
-    float dz = depth ? depth[idx] : 0.0f;
+    float len = sqrt_nr(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    view = make_float3(div_any(v[0], len), div_any(v[1], len), div_any(v[2], len));
     float wp[4];
     for (int row = 0; row < 4; ++row)
         wp[row] = D.ivp[0][row] * n0 + D.ivp[1][row] * n1 + D.ivp[2][row] * dz + D.ivp[3][row];
-    float3 world = make_float3(wp[0] / wp[3] * 1e-3f, wp[1] / wp[3] * 1e-3f, wp[2] / wp[3] * 1e-3f);
-    float3 rad, tr;
-    sky_radiance_to_point<H>(P, T, S, make_float3(D.cam[0], D.cam[1], D.cam[2]), view, world,
-                          make_float3(D.sun[0], D.sun[1], D.sun[2]), rad, tr);
+    world = make_float3(div_any(wp[0], wp[3]) * 1e-3f, div_any(wp[1], wp[3]) * 1e-3f,
+                        div_any(wp[2], wp[3]) * 1e-3f);
+}
+__device__ __forceinline__ void store_pixel(float4* __restrict__ color,
+                                            float4* __restrict__ trans_out, size_t idx,
+                                            int composite, float3 rad, float3 tr) {
     if (composite) {
         // Dual-source blend dst = src0 + dst * src1 (src/render.rs:124-136);
         // alpha: dst.a kept (src factor ZERO, dst factor ONE).
@@ -362,7 +570,93 @@ __global__ __launch_bounds__(256) void k_render_sky(DevParams P, const float4* _
 }
 
 template <bool H>
-__global__ __launch_bounds__(256) void k_render_rays(DevParams P, const float4* __restrict__ T,
+__global__ __launch_bounds__(256) void k_render_sky(DevParams P, SkyLut L, const float4* __restrict__ T,
+                                                    const float4* __restrict__ S, DrawArgs D,
+                                                    const float* __restrict__ depth, int w, int h,
+                                                    float4* __restrict__ color,
+                                                    float4* __restrict__ trans_out,
+                                                    int composite) {
+    int px = blockIdx.x * 16 + (threadIdx.x % 16);
+    int py = blockIdx.y * 16 + (threadIdx.x / 16);
+    if (px >= w || py >= h) return;
+    size_t idx = size_t(py) * w + px;
+    float3 view, world, rad, tr;
+    unproject(D, px, py, w, h, depth ? depth[idx] : 0.0f, view, world);
+    sky_radiance_to_point<H>(P, L, T, S, make_float3(D.cam[0], D.cam[1], D.cam[2]), view, world,
+                          make_float3(D.sun[0], D.sun[1], D.sun[2]), rad, tr);
+    store_pixel(color, trans_out, idx, composite, rad, tr);
+}
+
+// The draw's LUT slice at the camera's (r, mu_s), into `out`.
+template <bool H>
+__global__ __launch_bounds__(256) void k_draw_slice(DevParams P, const float4* __restrict__ T,
+                                                    const float4* __restrict__ S, float r,
+                                                    float mu_s, float4* __restrict__ out) {
+    build_sky_slice<H>(P, T, S, r, mu_s, out, int(blockIdx.x * blockDim.x + threadIdx.x),
+                       int(gridDim.x * blockDim.x));
+}
+// k_render_sky for a camera inside the atmosphere: every pixel starts at the
+// camera's r and mu_s, so the lookups there read the draw's slice (4 + 2 taps
+// from a table that fits the L1, not 16 + 4 from the LUTs, and no r and mu_s
+// coordinates), and a pixel with no geometry (depth 0) needs no others.
+// Bound by arithmetic and its latency (813 VALU instructions per pixel, 4 waves
+// per SIMD; 36 bytes of a pixel's traffic would take 15 us at 1080p): 54 us,
+// 101 us with IEEE divisions and square roots throughout and both lookups from
+// the LUTs.
+// smooth: smoothstep(0, 0.01, mu_s) (render_sky.h:182).
+template <bool H>
+__global__ __launch_bounds__(256) void k_render_sky_slice(
+    DevParams P, SkyLut L, SliceConsts C, float mu_s, float smooth, const float4* __restrict__ T,
+    const float4* __restrict__ S, const float4* __restrict__ slice, DrawArgs D,
+    const float* __restrict__ depth, int w, int h, float4* __restrict__ color,
+    float4* __restrict__ trans_out, int composite) {
+    int px = blockIdx.x * 16 + (threadIdx.x % 16);
+    int py = blockIdx.y * 16 + (threadIdx.x / 16);
+    if (px >= w || py >= h) return;
+    size_t idx = size_t(py) * w + px;
+    float3 view, world;
+    unproject(D, px, py, w, h, depth ? depth[idx] : 0.0f, view, world);
+    const float3 camera = make_float3(D.cam[0], D.cam[1], D.cam[2]),
+                 sun = make_float3(D.sun[0], D.sun[1], D.sun[2]);
+    // sky_radiance_to_point (render_sky.h:111-191)
+    const float r = C.r;
+    const float mu = div_rn(dot3(camera, view), r, C.r_inv);
+    const float nu = dot3(view, sun);
+    const bool ground = ray_intersects_ground<float>(P, r, mu);
+    const float3 pc =
+        make_float3(world.x - camera.x, world.y - camera.y, world.z - camera.z);
+    const float d = sqrtf(dot3(pc, pc));
+    const bool far_away = isinf(d);
+    const float r_p =
+        fminf(fmaxf(sqrt_nr(d * d + 2.0f * r * mu * d + r * r), L.bottom), L.top);
+    const float mu_p = far_away ? d : div_nr(r * mu + d, r_p);
+    float4 sc = slice_scattering(C, slice, P.s_nu, P.s_mu, mu, nu, ground);
+    const float mu_d = clamp_cosine<float>(mu_p);
+    const float3 far = lut_transmittance(L, T, far_away ? L.top : r_p, ground ? -mu_d : mu_d);
+    const float3 near = slice_transmittance(C, slice + (P.s_nu + 1) * P.s_mu, P.t_mu,
+                                            ground ? -mu : mu);
+    const float3 tr = lut_ratio(ground ? far : near, ground ? near : far);
+    float haze = 1.0f;
+    if (!far_away) {
+        const float4 sc_p = lut_scattering<H>(L, S, r_p, mu_p, div_nr(r * mu_s + d * nu, r_p), nu,
+                                              ground);
+        const float mr = single_mie_red(L, sc) - tr.x * single_mie_red(L, sc_p);
+        sc = make_float4(sc.x - tr.x * sc_p.x, sc.y - tr.y * sc_p.y, sc.z - tr.z * sc_p.z, mr);
+        haze = smooth;
+    }
+    float3 mie = extrapolated_single_mie(L, sc);
+    mie = make_float3(mie.x * haze, mie.y * haze, mie.z * haze);
+    const float pr = phase_rayleigh(nu), pm = lut_phase_mie(L, nu);
+    store_pixel(color, trans_out, idx, composite,
+                make_float3(sc.x * pr + mie.x * pm, sc.y * pr + mie.y * pm, sc.z * pr + mie.z * pm),
+                tr);
+}
+
+// Bound by the texture path of its scattered taps (TA busy 0.9 of the time):
+// with binary16 LUTs the two x neighbours of a tap pair come in one load, 8
+// instead of 16 per ray (4M random rays 242 -> 181 us).
+template <bool H>
+__global__ __launch_bounds__(256) void k_render_rays(DevParams P, SkyLut L, const float4* __restrict__ T,
                                                      const float4* __restrict__ S,
                                                      const float* __restrict__ cams, int cstride,
                                                      const float* __restrict__ views,
@@ -381,9 +675,9 @@ __global__ __launch_bounds__(256) void k_render_rays(DevParams P, const float4* 
     float3 rad, tr;
     if (points) {
         float3 pt = make_float3(points[3 * i], points[3 * i + 1], points[3 * i + 2]);
-        sky_radiance_to_point<H, true>(P, T, S, cam, view, pt, sun, rad, tr, l);
+        sky_radiance_to_point<H, true>(P, L, T, S, cam, view, pt, sun, rad, tr, l);
     } else {
-        sky_radiance<H, true>(P, T, S, cam, view, sun, rad, tr, l);
+        sky_radiance<H, true>(P, L, T, S, cam, view, sun, rad, tr, l);
     }
     rad_out[i] = make_float4(rad.x, rad.y, rad.z, 0.0f);
     if (trans_out) trans_out[i] = make_float4(tr.x, tr.y, tr.z, 1.0f);
@@ -506,6 +800,7 @@ __device__ void render_frame_block(const DevParams& P, const float4* __restrict_
     const FrameView v = frame_view(P, alt, zs);
     const float3 cam = v.cam, sun = v.sun;
     const float r = v.r;
+    const SkyLut L = sky_lut(P);
     SliceConsts sc;
     if constexpr (SLICE) {
         if (frame_slice) {
@@ -527,7 +822,7 @@ __device__ void render_frame_block(const DevParams& P, const float4* __restrict_
         if constexpr (SLICE)
             sky_radiance_slice(P, sc, s_slice, cam, view, sun, rad, tr);
         else
-            sky_radiance<H>(P, T, S, cam, view, sun, rad, tr);
+            sky_radiance<H>(P, L, T, S, cam, view, sun, rad, tr);
         const size_t o = size_t(frame) * pixels + p;  // frame-major output
         // Written once and not read back by the kernel: non-temporal stores.
         typedef float v4f __attribute__((ext_vector_type(4)));
@@ -676,13 +971,47 @@ fb_status fb_render_sky(fb_builder* b, fb_stream stream, const fb_atmosphere* ac
     auto* c4 = reinterpret_cast<float4*>(color);
     auto* t4 = reinterpret_cast<float4*>(transmittance);
     const int comp = int(flags & FB_RENDER_COMPOSITE);
-    if (a->dev.flags & fbk::kFlagF16Storage)
-        fbk::k_render_sky<true><<<grid, 256, 0, s>>>(a->dev, a->T.p, a->S.p, D, depth, int(width),
-                                                      int(height), c4, t4, comp);
+    const fbk::SkyLut L = fbk::sky_lut(a->dev);
+    const bool h = a->dev.flags & fbk::kFlagF16Storage;
+    // The camera's r and mu_s as the kernels compute them.
+    const float r = sqrtf(D.cam[0] * D.cam[0] + D.cam[1] * D.cam[1] + D.cam[2] * D.cam[2]);
+    const float mu_s =
+        (D.cam[0] * D.sun[0] + D.cam[1] * D.sun[1] + D.cam[2] * D.sun[2]) / r;
+    if (!(size_t(width) * height >= fbk::kDrawSliceMinPixels && r > 0.0f &&
+          r < a->dev.top * (1.0f - 1e-6f))) {
+#define FB_DRAW(H)                                                                             \
+    fbk::k_render_sky<H><<<grid, 256, 0, s>>>(a->dev, L, a->T.p, a->S.p, D, depth, int(width), \
+                                              int(height), c4, t4, comp)
+        h ? FB_DRAW(true) : FB_DRAW(false);
+#undef FB_DRAW
+        return end_use(a, s);
+    }
+    float4* slice = nullptr;
+    hipError_t e =
+        hipMallocAsync(reinterpret_cast<void**>(&slice), fbk::sky_slice_bytes(a->dev), s);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        set_error("draw slice scratch: %s", hipGetErrorString(e));
+        return e == hipErrorOutOfMemory ? FB_ENOMEM : FB_EHIP;
+    }
+    const unsigned sb = unsigned((fbk::sky_slice_float4s(a->dev) + 255) / 256);
+    const fbk::SliceConsts C = fbk::slice_consts(a->dev, r);
+    const float t = fminf(fmaxf(mu_s / 0.01f, 0.0f), 1.0f), smooth = t * t * (3.0f - 2.0f * t);
+#define FB_DRAW(H)                                                                               \
+    do {                                                                                         \
+        fbk::k_draw_slice<H><<<sb, 256, 0, s>>>(a->dev, a->T.p, a->S.p, r, mu_s, slice);         \
+        fbk::k_render_sky_slice<H><<<grid, 256, 0, s>>>(a->dev, L, C, mu_s, smooth, a->T.p,      \
+                                                        a->S.p, slice, D, depth, int(width),     \
+                                                        int(height), c4, t4, comp);              \
+    } while (0)
+    if (h)
+        FB_DRAW(true);
     else
-        fbk::k_render_sky<false><<<grid, 256, 0, s>>>(a->dev, a->T.p, a->S.p, D, depth,
-                                                       int(width), int(height), c4, t4, comp);
-    return end_use(a, s);
+        FB_DRAW(false);
+#undef FB_DRAW
+    e = hipGetLastError();
+    const hipError_t fe = hipFreeAsync(slice, s);
+    return end_use(a, s, e == hipSuccess ? fe : e);
 }
 
 fb_status fb_render_sky_rays_shadowed(fb_builder* b, fb_stream stream, const fb_atmosphere* ac,
@@ -702,15 +1031,16 @@ fb_status fb_render_sky_rays_shadowed(fb_builder* b, fb_stream stream, const fb_
     hipStream_t s = static_cast<hipStream_t>(stream);
     if ((st = begin_use(a, s)) != FB_OK) return st;
     const unsigned blocks = unsigned((n + 255) / 256);
+    const fbk::SkyLut L = fbk::sky_lut(a->dev);
     auto* r4 = reinterpret_cast<float4*>(radiance);
     auto* t4 = reinterpret_cast<float4*>(transmittance);
     if (a->dev.flags & fbk::kFlagF16Storage)
-        fbk::k_render_rays<true><<<blocks, 256, 0, s>>>(a->dev, a->T.p, a->S.p, cameras,
+        fbk::k_render_rays<true><<<blocks, 256, 0, s>>>(a->dev, L, a->T.p, a->S.p, cameras,
                                                          int(camera_stride), views, points, suns,
                                                          int(sun_stride), shadow_lengths, n, r4,
                                                          t4);
     else
-        fbk::k_render_rays<false><<<blocks, 256, 0, s>>>(a->dev, a->T.p, a->S.p, cameras,
+        fbk::k_render_rays<false><<<blocks, 256, 0, s>>>(a->dev, L, a->T.p, a->S.p, cameras,
                                                           int(camera_stride), views, points, suns,
                                                           int(sun_stride), shadow_lengths, n, r4,
                                                           t4);
