@@ -165,9 +165,10 @@ fb_status add_launch(BatchPlan& plan, const std::vector<fb_parameters>& ps,
                      const std::vector<fbk::DevParams>& dps, const std::vector<fbk::Tuning>& tus,
                      const std::vector<int>& order_idx, int pass, int order) {
     auto member = [&](int i) { return pass < fbk::kPassDensity || int(ps[i].order) >= order; };
-    // One launch per block shape.  Multiple scattering: each atmosphere runs
-    // its own tuned shape (rows of very different widths want different
-    // block sizes), one launch per distinct (threads, texels per thread).
+    // One launch per block shape.  Multiple scattering and density: each
+    // atmosphere runs its own shape (rows and tiles of very different widths
+    // want different block sizes), one launch per distinct (threads, texels
+    // per thread).
     // The other tunable passes: one launch, with the tuning of its largest
     // atmosphere when that suits every member, else a size that suits all.
     struct Group {
@@ -207,13 +208,13 @@ fb_status add_launch(BatchPlan& plan, const std::vector<fb_parameters>& ps,
             else
                 g->members.push_back(i);
         } else if (pass == fbk::kPassDensity) {
-            // One launch per texels-per-thread variant (den_tpx).
+            // One launch per block size and texels-per-thread variant (den_tpx).
+            const unsigned t = fbk::tuned_threads(dps[i], pass, order, tus[i]);
             const unsigned c = unsigned(fbk::den_tpx(dps[i]));
             auto g = std::find_if(groups.begin(), groups.end(),
-                                  [&](const Group& x) { return x.tpt == c; });
+                                  [&](const Group& x) { return x.threads == t && x.tpt == c; });
             if (g == groups.end())
-                groups.push_back(Group{fbk::tuned_threads(dps[i], pass, order, tus[i]), c,
-                                       bool((tus[i].remap >> pass) & 1u), {i}});
+                groups.push_back(Group{t, c, bool((tus[i].remap >> pass) & 1u), {i}});
             else
                 g->members.push_back(i);
         } else if (groups.empty()) {
@@ -223,7 +224,7 @@ fb_status add_launch(BatchPlan& plan, const std::vector<fb_parameters>& ps,
             groups[0].members.push_back(i);
         }
     }
-    if (tunable && pass != fbk::kPassMultiple)
+    if (tunable && pass != fbk::kPassMultiple && pass != fbk::kPassDensity)
         for (Group& g : groups)
             for (int i : g.members)
                 if (!fbk::tuning_valid(dps[i], pass, order, g.threads))

@@ -11,6 +11,9 @@
 // bit-identical LUTs; plain and batched builds read the same table.
 #include <string.h>
 
+#include <algorithm>
+#include <iterator>
+
 #include "runtime.hpp"
 
 namespace fbrt {
@@ -116,17 +119,28 @@ fb_status fb_builder_autotune(fb_builder* b, fb_stream stream, const fb_paramete
                     int remap_pass, auto launch) -> fb_status {
         float best_t = -1.0f;
         unsigned best_v = 0;
-        for (unsigned c : candidates) {
-            if (!fbk::tuning_valid(P, pass, order, c)) continue;
+        auto try_size = [&](unsigned c) -> fb_status {
+            if (!fbk::tuning_valid(P, pass, order, c)) return FB_OK;
             fbk::Tuning t = best;
             t.*field = c / unit;
             float ms = 0.0f;
             fb_status st2 = time(t, launch, &ms);
-            if (st2 != FB_OK) return st2;
-            if (best_t < 0.0f || ms < best_t) {
+            if (st2 == FB_OK && (best_t < 0.0f || ms < best_t)) {
                 best_t = ms;
                 best_v = c / unit;
             }
+            return st2;
+        };
+        for (unsigned c : candidates) {
+            fb_status st2 = try_size(c);
+            if (st2 != FB_OK) return st2;
+        }
+        // The density tile's own block size, where that is none of them.
+        const unsigned own = fbk::default_threads(P, pass, order);
+        if (pass == fbk::kPassDensity &&
+            std::find(std::begin(candidates), std::end(candidates), own) == std::end(candidates)) {
+            fb_status st2 = try_size(own);
+            if (st2 != FB_OK) return st2;
         }
         if (!best_v) return FB_OK;
         best.*field = best_v;
