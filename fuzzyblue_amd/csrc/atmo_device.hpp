@@ -105,11 +105,24 @@ __device__ __forceinline__ G smoothstep_g(G e0, G e1, G x) {
     return t * t * (G(3) - G(2) * t);
 }
 
+// a / b correctly rounded, given y = 1/b correctly rounded and b normal: q =
+// a*y, then Markstein's correction q + (a - b*q)*y with the residual exact
+// in an FMA (P. Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", IBM J. Res. Dev. 34(1), 1990) -- three
+// instructions in place of an IEEE division's ten, the same bits while a is 0
+// or at least 2^-80 (the residual is a multiple of about 2^(e_a - 46)).
+__device__ __forceinline__ float div_markstein(float a, float b, float y) {
+    const float q = a * y;
+    return fmaf(fmaf(-q, b, a), y, q);
+}
+
 // -------------------------------------------------------------- params.h
 // params.h:89-93 (altitude in FP32, as the density value is FP32)
 __device__ __forceinline__ float layer_density(const DevLayer& l, float altitude) {
-    float density = l.exp_term * expf(l.exp_scale * altitude) + l.linear_term * altitude +
-                    l.constant_term;
+    // (A layer without an exponential, as the ozone tent's, skips it: exp(0) is
+    // 1 and the branch is uniform.)
+    const float e = l.exp_scale == 0.0f ? 1.0f : expf(l.exp_scale * altitude);
+    float density = l.exp_term * e + l.linear_term * altitude + l.constant_term;
     return fminf(fmaxf(density, 0.0f), 1.0f);
 }
 // params.h:95-99

@@ -165,10 +165,10 @@ fb_status add_launch(BatchPlan& plan, const std::vector<fb_parameters>& ps,
                      const std::vector<fbk::DevParams>& dps, const std::vector<fbk::Tuning>& tus,
                      const std::vector<int>& order_idx, int pass, int order) {
     auto member = [&](int i) { return pass < fbk::kPassDensity || int(ps[i].order) >= order; };
-    // One launch per block shape.  Multiple scattering and density: each
-    // atmosphere runs its own shape (rows and tiles of very different widths
-    // want different block sizes), one launch per distinct (threads, texels
-    // per thread).
+    // One launch per block shape.  Single and multiple scattering and density:
+    // each atmosphere runs its own shape (rows and tiles of very different
+    // widths want different block sizes), one launch per distinct (threads,
+    // texels per thread).
     // The other tunable passes: one launch, with the tuning of its largest
     // atmosphere when that suits every member, else a size that suits all.
     struct Group {
@@ -182,18 +182,19 @@ fb_status add_launch(BatchPlan& plan, const std::vector<fb_parameters>& ps,
     for (int i : order_idx) {
         if (!member(i)) continue;
         if (pass == fbk::kPassSingle) {
-            // The staged kernel (transmittance rows in LDS), the direct one,
-            // or the chunked direct one for narrow rows: one launch per kernel.
-            const unsigned c = fbk::ss_chunked(dps[i])  ? fbk::kSsChunked
-                               : fbk::ss_staged(dps[i]) ? fbk::kSsStaged
+            // The staged kernel (transmittance rows in LDS) by its texels per
+            // thread, the direct one, or the chunked direct one for narrow
+            // rows: one launch per kernel and block size.
+            const bool chunked = fbk::ss_chunked(dps[i]);
+            const unsigned t = chunked ? fbk::kSsChunkThreads
+                                       : fbk::tuned_threads(dps[i], pass, order, tus[i]);
+            const unsigned c = chunked                  ? fbk::kSsChunked
+                               : fbk::ss_staged(dps[i]) ? fbk::ss_tpt(dps[i], t)
                                                         : fbk::kSsDirect;
             auto g = std::find_if(groups.begin(), groups.end(),
-                                  [&](const Group& x) { return x.tpt == c; });
+                                  [&](const Group& x) { return x.threads == t && x.tpt == c; });
             if (g == groups.end())
-                groups.push_back(Group{c == fbk::kSsChunked
-                                           ? fbk::kSsChunkThreads
-                                           : fbk::tuned_threads(dps[i], pass, order, tus[i]),
-                                       c, bool((tus[i].remap >> pass) & 1u), {i}});
+                groups.push_back(Group{t, c, bool((tus[i].remap >> pass) & 1u), {i}});
             else
                 g->members.push_back(i);
         } else if (pass == fbk::kPassMultiple) {
@@ -224,11 +225,10 @@ fb_status add_launch(BatchPlan& plan, const std::vector<fb_parameters>& ps,
             groups[0].members.push_back(i);
         }
     }
-    if (tunable && pass != fbk::kPassMultiple && pass != fbk::kPassDensity)
+    if (pass == fbk::kPassIndirect)
         for (Group& g : groups)
             for (int i : g.members)
-                if (!fbk::tuning_valid(dps[i], pass, order, g.threads))
-                    g.threads = pass == fbk::kPassIndirect ? 64 : 256;
+                if (!fbk::tuning_valid(dps[i], pass, order, g.threads)) g.threads = 64;
     for (Group& g : groups) {
         BatchLaunch l;
         l.pass = pass;

@@ -222,9 +222,15 @@ inline bool ss_chunked(const DevParams& P) {
 inline size_t ss_chunked_lds_bytes(const DevParams& P) {
     return 24 * size_t(ss_chunks(P)) * size_t(P.s_nu * P.s_mus);
 }
-// The kernel code of a batched single-scattering launch: staged, direct
-// lookups, or chunked direct lookups.
-constexpr unsigned kSsDirect = 0, kSsStaged = 1, kSsChunked = 2;
+// Staged texels per thread for blocks of `threads` (1, 2 or 4): registers of
+// texels a thread does not have cost occupancy.
+inline unsigned ss_tpt(const DevParams& P, unsigned threads) {
+    const unsigned w = unsigned(P.s_nu * P.s_mus);
+    return w <= threads ? 1u : (w <= 2 * threads ? 2u : unsigned(kSsTexelsPerThread));
+}
+// The kernel code of a batched single-scattering launch: the staged texels
+// per thread, direct lookups, or chunked direct lookups.
+constexpr unsigned kSsDirect = 0, kSsChunked = 8;
 
 unsigned tuned_threads(const DevParams& P, int pass, int order, const Tuning& tu);
 bool tuning_valid(const DevParams& P, int pass, int order, unsigned threads);

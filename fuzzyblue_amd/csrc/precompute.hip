@@ -178,13 +178,16 @@ __device__ __forceinline__ void transmittance_block_ordered(const DevParams& P, 
         s_terms[wave][1][k] = profile_density(P.prof[1], alt) * w * dxf;
         s_terms[wave][2][k] = profile_density(P.prof[2], alt) * w * dxf;
     }
+    // The first wavefront sums the block's four texels, one lane per texel and
+    // profile: a quarter of the issue slots of each wavefront summing its own.
+    __shared__ float s_len[12];
     __syncthreads();
-    float L = 0.0f;
-    if (lane < 3) {
+    if (threadIdx.x < 12) {
         // Terms 0..499 four at a time (still added one by one, in order),
         // then term 500.
-        const float* tp = s_terms[wave][lane];
+        const float* tp = s_terms[threadIdx.x / 3][threadIdx.x % 3];
         const float4* tp4 = reinterpret_cast<const float4*>(tp);
+        float L = 0.0f;
 #pragma unroll 5
         for (int q = 0; q < SAMPLE_COUNT / 4; ++q) {
             const float4 v = tp4[q];
@@ -193,10 +196,11 @@ __device__ __forceinline__ void transmittance_block_ordered(const DevParams& P, 
             L = L + v.z;
             L = L + v.w;
         }
-        L = L + tp[SAMPLE_COUNT];
+        s_len[threadIdx.x] = L + tp[SAMPLE_COUNT];
     }
-    const float LR = __shfl(L, 0, 64), LM = __shfl(L, 1, 64), LO = __shfl(L, 2, 64);
+    __syncthreads();
     if (!active || lane != 0) return;
+    const float LR = s_len[3 * wave], LM = s_len[3 * wave + 1], LO = s_len[3 * wave + 2];
     store_transmittance(P, i, j, LR, LM, LO, T, nullptr);
 }
 
@@ -394,10 +398,12 @@ __device__ __forceinline__ void ss_sun_coord(float rf, float mu_s, float nu, flo
         // tex_from_unit then linear_taps: texel coordinate x_mu*(N-1).
         t = __builtin_amdgcn_fmed3f((d - lq.y) * iv.y * tmax, 0.0f, tmax);
     } else {
-        mu_s_d = clamp_cosine<float>((rf * mu_s + d_i * nu) / r_d);
+        // (The table's reciprocals are IEEE ones here: the quotients' bits are
+        // the divisions'.)
+        mu_s_d = clamp_cosine<float>(div_markstein(rf * mu_s + d_i * nu, r_d, iv.x));
         float disc = r_d * r_d * (mu_s_d * mu_s_d - 1.0f) + top2;
         float d = clamp_distance<float>(-r_d * mu_s_d + safe_sqrt<float>(disc));
-        float x_mu = (d - lq.y) / lq.z;
+        float x_mu = div_markstein(d - lq.y, lq.z, iv.y);
         // linear_taps of tex_from_unit(x_mu): u*N - 0.5 = x_mu*(N-1), clamped.
         const float u = tex_from_unit<float>(x_mu, TMU);
         t = fminf(fmaxf(u * float(TMU) - 0.5f, 0.0f), tmax);
@@ -409,14 +415,20 @@ __device__ __forceinline__ void ss_sun_coord(float rf, float mu_s, float nu, flo
 }
 
 
-// STAGED: per sample, the block first interpolates the sample's two
-// transmittance rows (its r taps) into one row in LDS (double buffered, one
-// barrier per sample) and each texel interpolates that row in mu: all
-// texels of the (r, mu) row look up the same two LUT rows, so this replaces
-// four scattered loads per texel and sample by coalesced loads of the rows.
-// Otherwise (transmittance LUTs wider than kSsMaxStagedMu) each texel reads
-// its four taps itself.
-template <typename G, bool COMP, bool H, bool STAGED>
+// STAGED (texels per thread): per sample, the block first interpolates the
+// sample's two transmittance rows (its r taps) into one row in LDS (double
+// buffered, one barrier per sample) and each texel interpolates that row in
+// mu: all texels of the (r, mu) row look up the same two LUT rows, so this
+// replaces four scattered loads per texel and sample by coalesced loads of the
+// rows.  0 (transmittance LUTs wider than kSsMaxStagedMu): each texel reads its
+// four taps itself.
+//
+// Staged it is bound by the chain of a sample and its LDS taps, which scatter
+// over the row (half of the LDS cycles are bank conflicts).  With the rows
+// loaded and staged before the evaluation, registers for four texels in every
+// thread and IEEE divisions in FP32 mode: default 0.125 ms, now 0.120 (FP32
+// mode 0.177, now 0.151), double 1.16, now 1.09, 27x64x26x18 0.093, now 0.087.
+template <typename G, bool COMP, bool H, int STAGED>
 __device__ __forceinline__ void single_scattering_block(const DevParams& P, const int bx, const int by, const int bz,
                                                            const float4* __restrict__ T,
                                                            const float4* __restrict__ SR,
@@ -458,6 +470,15 @@ __device__ __forceinline__ void single_scattering_block(const DevParams& P, cons
     auto accumulate = [&](Sum<COMP>* rs, Sum<COMP>* ms, float4 tv, float4 gq, float3 ts,
                           float sm) {
         float t0 = tv.x * (ts.x * sm), t1 = tv.y * (ts.y * sm), t2 = tv.z * (ts.z * sm);
+        if constexpr (kPrecise && !COMP) {
+            rs[0].s = fmaf(t0, gq.y, rs[0].s);
+            rs[1].s = fmaf(t1, gq.y, rs[1].s);
+            rs[2].s = fmaf(t2, gq.y, rs[2].s);
+            ms[0].s = fmaf(t0, gq.z, ms[0].s);
+            ms[1].s = fmaf(t1, gq.z, ms[1].s);
+            ms[2].s = fmaf(t2, gq.z, ms[2].s);
+            return;
+        }
         rs[0].add(t0 * gq.y);
         rs[1].add(t1 * gq.y);
         rs[2].add(t2 * gq.y);
@@ -465,12 +486,12 @@ __device__ __forceinline__ void single_scattering_block(const DevParams& P, cons
         ms[1].add(t1 * gq.z);
         ms[2].add(t2 * gq.z);
     };
-    if constexpr (STAGED) {
+    if constexpr (STAGED != 0) {
         extern __shared__ float4 s_trow[];  // [2][TMU]
-        float tmu_s[kSsTexelsPerThread], tnu[kSsTexelsPerThread];
-        Sum<COMP> rs[kSsTexelsPerThread][3], ms[kSsTexelsPerThread][3];
+        float tmu_s[STAGED], tnu[STAGED];
+        Sum<COMP> rs[STAGED][3], ms[STAGED][3];
 #pragma unroll
-        for (int q = 0; q < kSsTexelsPerThread; ++q) {
+        for (int q = 0; q < STAGED; ++q) {
             const int x = tid + q * nt;
             tmu_s[q] = 0.0f;
             tnu[q] = 0.0f;
@@ -481,26 +502,56 @@ __device__ __forceinline__ void single_scattering_block(const DevParams& P, cons
                 tnu[q] = float(c.nu);
             }
         }
-        // Sample i's two T rows, lerped in r with the row weight, into dst.
-        auto stage = [&](int i, float4* dst) {
+        // Sample i's two T rows, lerped in r with the row weight, into a staged
+        // row.  The first kAhead columns of a thread are loaded before the
+        // evaluation of the sample before and written after it, so that their
+        // latency is hidden; further ones at once.
+        constexpr int kAhead = 2;
+        float3 ta[kAhead], tb[kAhead];
+        auto load = [&](int i) {
             const float4 tr4 = s_trw[i];
-            const float w = s_lut[i].w;
             const float4* t0 = T + __float_as_int(tr4.x);
             const float4* t1 = T + __float_as_int(tr4.y);
-            for (int j = tid; j < TMU; j += nt) {
-                const float4 a = ldg4(t0 + j), b = ldg4(t1 + j);
-                dst[j] = make_float4(fmaf(w, b.x - a.x, a.x), fmaf(w, b.y - a.y, a.y),
-                                     fmaf(w, b.z - a.z, a.z), 0.0f);
+#pragma unroll
+            for (int c = 0; c < kAhead; ++c) {
+                const int j = tid + c * nt;
+                if (j < TMU) {
+                    ta[c] = *reinterpret_cast<const float3*>(t0 + j);
+                    tb[c] = *reinterpret_cast<const float3*>(t1 + j);
+                }
             }
         };
-        stage(0, s_trow);
+        auto put = [&](int i, float4* dst) {
+            const float w = s_lut[i].w;
+#pragma unroll
+            for (int c = 0; c < kAhead; ++c) {
+                const int j = tid + c * nt;
+                if (j < TMU) {
+                    const float3 v = lerp3(ta[c], tb[c], w);
+                    dst[j] = make_float4(v.x, v.y, v.z, 0.0f);
+                }
+            }
+            if (kAhead * nt < TMU) {
+                const float4 tr4 = s_trw[i];
+                const float4* t0 = T + __float_as_int(tr4.x);
+                const float4* t1 = T + __float_as_int(tr4.y);
+                for (int j = tid + kAhead * nt; j < TMU; j += nt) {
+                    const float4 a = ldg4(t0 + j), b = ldg4(t1 + j);
+                    dst[j] = make_float4(fmaf(w, b.x - a.x, a.x), fmaf(w, b.y - a.y, a.y),
+                                         fmaf(w, b.z - a.z, a.z), 0.0f);
+                }
+            }
+        };
+        load(0);
+        put(0, s_trow);
         __syncthreads();
         for (int i = 0; i < kMsSamples; ++i) {
             const float4* cur = s_trow + (i & 1) * TMU;
-            if (i + 1 < kMsSamples) stage(i + 1, s_trow + ((i + 1) & 1) * TMU);
+            const bool next = i + 1 < kMsSamples;
+            if (next) load(i + 1);
             const float4 tv = s_tv[i], gq = s_geo[i], lq = s_lut[i], iv = s_inv[i];
 #pragma unroll
-            for (int q = 0; q < kSsTexelsPerThread; ++q) {
+            for (int q = 0; q < STAGED; ++q) {
                 if (tid + q * nt >= W) continue;
                 float t, sm;
                 ss_sun_coord<kPrecise>(rf, tmu_s[q], tnu[q], tv, gq, lq, iv, top2, TMU, t, sm);
@@ -512,10 +563,11 @@ __device__ __forceinline__ void single_scattering_block(const DevParams& P, cons
                                               fmaf(f, b.z - a.z, a.z));
                 accumulate(rs[q], ms[q], tv, gq, ts, sm);
             }
+            if (next) put(i + 1, s_trow + ((i + 1) & 1) * TMU);
             __syncthreads();
         }
 #pragma unroll
-        for (int q = 0; q < kSsTexelsPerThread; ++q)
+        for (int q = 0; q < STAGED; ++q)
             if (tid + q * nt < W) store(tid + q * nt, rs[q], ms[q]);
     } else {
         for (int x = tid; x < W; x += nt) {
@@ -1343,7 +1395,7 @@ __global__ __launch_bounds__(256) void kb_direct_irradiance(const DevParams* __r
     }
 }
 
-template <typename G, bool COMP, bool H, bool STAGED>
+template <typename G, bool COMP, bool H, int STAGED>
 __global__ __launch_bounds__(256) void k_single_scattering(DevParams P, const float4* __restrict__ T,
                                                            const float4* __restrict__ SR,
                                                            float4* __restrict__ dR,
@@ -1353,7 +1405,7 @@ __global__ __launch_bounds__(256) void k_single_scattering(DevParams P, const fl
     const unsigned b = logical_block(remap);
     single_scattering_block<G, COMP, H, STAGED>(P, b % P.s_mu, b / P.s_mu, 0, T, SR, dR, dM, S);
 }
-template <typename G, bool COMP, bool H, bool STAGED>
+template <typename G, bool COMP, bool H, int STAGED>
 __global__ __launch_bounds__(256) void kb_single_scattering(const DevParams* __restrict__ Ps,
                                                             const LutPtrs* __restrict__ L,
                                                             const uint32_t* __restrict__ tiles, unsigned ntiles) {
@@ -1571,16 +1623,18 @@ static hipError_t launch_single_scattering_h(const DevParams& P, const float4* T
                 <<<grid, kSsChunkThreads, lds, s>>>(P, T, SR, dR, dM, S, remap);
     } else if (ss_staged(P)) {
         const size_t lds = ss_staged_lds_bytes(P.t_mu);
+        const unsigned tpt = ss_tpt(P, threads);
+#define FB_SS(G, X) \
+    k_single_scattering<G, false, H, X><<<grid, threads, lds, s>>>(P, T, SR, dR, dM, S, remap)
         if (P.flags & 1)
-            k_single_scattering<double, false, H, true>
-                <<<grid, threads, lds, s>>>(P, T, SR, dR, dM, S, remap);
+            tpt == 1 ? FB_SS(double, 1) : tpt == 2 ? FB_SS(double, 2) : FB_SS(double, 4);
         else
-            k_single_scattering<float, false, H, true>
-                <<<grid, threads, lds, s>>>(P, T, SR, dR, dM, S, remap);
+            tpt == 1 ? FB_SS(float, 1) : tpt == 2 ? FB_SS(float, 2) : FB_SS(float, 4);
+#undef FB_SS
     } else if (P.flags & 1) {
-        k_single_scattering<double, false, H, false><<<grid, threads, 0, s>>>(P, T, SR, dR, dM, S, remap);
+        k_single_scattering<double, false, H, 0><<<grid, threads, 0, s>>>(P, T, SR, dR, dM, S, remap);
     } else {
-        k_single_scattering<float, false, H, false><<<grid, threads, 0, s>>>(P, T, SR, dR, dM, S, remap);
+        k_single_scattering<float, false, H, 0><<<grid, threads, 0, s>>>(P, T, SR, dR, dM, S, remap);
     }
     return hipGetLastError();
 }
@@ -1791,20 +1845,25 @@ static hipError_t launch_batch_h(int pass, int order, bool precise, const DevPar
             else
                 kb_direct_irradiance<float><<<grid, block, 0, s>>>(Ps, L, tiles, ntiles);
             break;
-        case kPassSingle:  // tpt: kSsStaged, kSsDirect or kSsChunked
+        case kPassSingle:  // tpt: staged texels per thread, kSsDirect or kSsChunked
+#define FB_KBSS(G, X) kb_single_scattering<G, false, H, X><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles)
             if (tpt == kSsChunked) {
                 if (precise)
                     kb_single_scattering_chunked<double, H><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles);
                 else
                     kb_single_scattering_chunked<float, H><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles);
-            } else if (precise && tpt)
-                kb_single_scattering<double, false, H, true><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles);
-            else if (precise)
-                kb_single_scattering<double, false, H, false><<<grid, block, 0, s>>>(Ps, L, tiles, ntiles);
-            else if (tpt)
-                kb_single_scattering<float, false, H, true><<<grid, block, lds, s>>>(Ps, L, tiles, ntiles);
-            else
-                kb_single_scattering<float, false, H, false><<<grid, block, 0, s>>>(Ps, L, tiles, ntiles);
+            } else if (precise) {
+                tpt == 4   ? FB_KBSS(double, 4)
+                : tpt == 2 ? FB_KBSS(double, 2)
+                : tpt == 1 ? FB_KBSS(double, 1)
+                           : FB_KBSS(double, 0);
+            } else {
+                tpt == 4   ? FB_KBSS(float, 4)
+                : tpt == 2 ? FB_KBSS(float, 2)
+                : tpt == 1 ? FB_KBSS(float, 1)
+                           : FB_KBSS(float, 0);
+            }
+#undef FB_KBSS
             break;
         case kPassClear:
             kb_clear_irradiance<<<grid, block, 0, s>>>(Ps, L, tiles, ntiles);
@@ -1879,12 +1938,15 @@ static unsigned batch_resident_blocks_h(int pass, int order, bool precise, unsig
             if (tpt == kSsChunked)
                 fn = precise ? (const void*)kb_single_scattering_chunked<double, H>
                              : (const void*)kb_single_scattering_chunked<float, H>;
-            else if (tpt)
-                fn = precise ? (const void*)kb_single_scattering<double, false, H, true>
-                             : (const void*)kb_single_scattering<float, false, H, true>;
             else
-                fn = precise ? (const void*)kb_single_scattering<double, false, H, false>
-                             : (const void*)kb_single_scattering<float, false, H, false>;
+#define FB_KBSS(X)                                                        \
+    (precise ? (const void*)kb_single_scattering<double, false, H, X>     \
+             : (const void*)kb_single_scattering<float, false, H, X>)
+                fn = tpt == 4   ? FB_KBSS(4)
+                     : tpt == 2 ? FB_KBSS(2)
+                     : tpt == 1 ? FB_KBSS(1)
+                                : FB_KBSS(0);
+#undef FB_KBSS
             break;
         case kPassClear:
             fn = (const void*)kb_clear_irradiance;

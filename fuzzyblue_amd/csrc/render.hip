@@ -14,19 +14,12 @@ __device__ __forceinline__ float dot3(float3 a, float3 b) {
     return a.x * b.x + a.y * b.y + a.z * b.z;
 }
 
-// a / b correctly rounded, given y = 1/b correctly rounded and b normal: q =
-// a*y, then Markstein's correction q + (a - b*q)*y with the residual exact
-// in an FMA (P. Markstein, "Computation of elementary functions on the IBM
-// RISC System/6000 processor", IBM J. Res. Dev. 34(1), 1990) -- three
-// instructions in place of an IEEE division's ten, the same bits.  The
-// residual is a multiple of about 2^(e_a - 46): for numerators below 2^-80
-// (other than 0) it can be subnormal or not representable, and a wavefront
-// with such a lane takes the division (a wave-uniform branch; the empty asm
-// statement keeps the compiler from evaluating the division unconditionally
-// and selecting).
+// div_markstein for any numerator: a wavefront with a lane below 2^-80 (other
+// than 0) takes the division (a wave-uniform branch; the empty asm statement
+// keeps the compiler from evaluating the division unconditionally and
+// selecting).
 __device__ __forceinline__ float div_rn(float a, float b, float y) {
-    const float q = a * y;
-    float d = fmaf(fmaf(-q, b, a), y, q);
+    float d = div_markstein(a, b, y);
     if (__builtin_amdgcn_ballot_w64(a != 0.0f && fabsf(a) < 0x1p-80f)) {
         asm volatile("");
         d = a / b;
