@@ -970,22 +970,28 @@ fb_status fb_render_sky(fb_builder* b, fb_stream stream, const fb_atmosphere* ac
     const float r = sqrtf(D.cam[0] * D.cam[0] + D.cam[1] * D.cam[1] + D.cam[2] * D.cam[2]);
     const float mu_s =
         (D.cam[0] * D.sun[0] + D.cam[1] * D.sun[1] + D.cam[2] * D.sun[2]) / r;
-    if (!(size_t(width) * height >= fbk::kDrawSliceMinPixels && r > 0.0f &&
-          r < a->dev.top * (1.0f - 1e-6f))) {
+    // The slice covers what its clamps agree with the per-pixel lookups on: a
+    // camera in the atmosphere and a sun vector no longer than 1 (nu of longer
+    // ones leaves the LUT's range).  Where its scratch cannot be had, and in a
+    // captured draw (no allocations there), the draw looks the LUTs up.
+    float4* slice = nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (size_t(width) * height >= fbk::kDrawSliceMinPixels &&
+        r >= a->dev.bottom * (1.0f - 1e-6f) && r < a->dev.top * (1.0f - 1e-6f) &&
+        D.sun[0] * D.sun[0] + D.sun[1] * D.sun[1] + D.sun[2] * D.sun[2] <= 1.0f + 1e-5f &&
+        hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+        hipMallocAsync(reinterpret_cast<void**>(&slice), fbk::sky_slice_bytes(a->dev), s) !=
+            hipSuccess) {
+        (void)hipGetLastError();
+        slice = nullptr;
+    }
+    if (!slice) {
 #define FB_DRAW(H)                                                                             \
     fbk::k_render_sky<H><<<grid, 256, 0, s>>>(a->dev, L, a->T.p, a->S.p, D, depth, int(width), \
                                               int(height), c4, t4, comp)
         h ? FB_DRAW(true) : FB_DRAW(false);
 #undef FB_DRAW
         return end_use(a, s);
-    }
-    float4* slice = nullptr;
-    hipError_t e =
-        hipMallocAsync(reinterpret_cast<void**>(&slice), fbk::sky_slice_bytes(a->dev), s);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        set_error("draw slice scratch: %s", hipGetErrorString(e));
-        return e == hipErrorOutOfMemory ? FB_ENOMEM : FB_EHIP;
     }
     const unsigned sb = unsigned((fbk::sky_slice_float4s(a->dev) + 255) / 256);
     const fbk::SliceConsts C = fbk::slice_consts(a->dev, r);
@@ -1002,8 +1008,7 @@ fb_status fb_render_sky(fb_builder* b, fb_stream stream, const fb_atmosphere* ac
     else
         FB_DRAW(false);
 #undef FB_DRAW
-    e = hipGetLastError();
-    const hipError_t fe = hipFreeAsync(slice, s);
+    const hipError_t e = hipGetLastError(), fe = hipFreeAsync(slice, s);
     return end_use(a, s, e == hipSuccess ? fe : e);
 }
 

@@ -1,0 +1,63 @@
+"""Draws large enough for the per-draw LUT slice (1500 x 1001 pixels, which
+fill no block evenly) against the FP32 restatement of render_sky.frag:24-35,
+with and without geometry behind each pixel, and the same draw with a sun
+vector longer than 1, which the slice does not cover.
+
+Tolerances are those of the small draw's comparison (transmittance 1e-4 at a
+floor of 1e-6 of the maximum, radiance 1e-3 at 1e-4).  One pixel in a thousand
+may exceed them: the horizon, one row of the 1001, is where an ulp of the view
+direction moves a lookup between the two halves of the scattering LUT.
+"""
+import numpy as np
+import pytest
+
+from fuzzyblue_amd import (Atmosphere, DeviceBuffer, DrawParameters, Parameters, Renderer,
+                           synchronize)
+from fuzzyblue_amd.params import DUMP_SIZES
+from oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+W, H = 1500, 1001
+
+
+def rel_err(x, y, floor):
+    x = np.asarray(x, np.float64)[..., :3]
+    y = np.asarray(y, np.float64)[..., :3]
+    return np.abs(x - y) / np.maximum(np.abs(y), floor * max(np.abs(y).max(), 1e-30))
+
+
+@pytest.mark.parametrize("sun_length", [1.0, 1.01])
+def test_large_draw_matches_fragment_shader(builder, sun_length):
+    p = Parameters().replace(**DUMP_SIZES)
+    pa = Atmosphere.build(builder, None, p)
+    pa.wait()
+    a = pa.assert_ready()
+    T = a.download("transmittance").astype(np.float64)
+    S = a.download("scattering").astype(np.float64)
+    # Inverse of a reverse-Z infinite perspective for a camera 2 km up looking
+    # along +x (column-major, [column][row]), in metres.
+    near = 0.1
+    ivp = np.zeros((4, 4), np.float32)
+    ivp[0] = [0.0, -0.75, 0.0, 0.0]
+    ivp[1] = [0.0, 0.0, -0.5, 0.0]
+    ivp[2] = [0.0, 0.0, 6362e3 / near, 1.0 / near]
+    ivp[3] = [1.0, 0.0, 0.0, 0.0]
+    draw = DrawParameters(inverse_viewproj=ivp.tolist(), camera_position=[0.0, 0.0, 6362.0],
+                          sun_direction=[0.6 * sun_length, 0.0, 0.8 * sun_length])
+    depth = np.random.default_rng(3).uniform(near / 50e3, near / 500.0, (H, W)).astype(np.float32)
+    depth[: H // 2] = 0.0  # upper half: infinitely far
+    color, tr = DeviceBuffer(W * H * 16), DeviceBuffer(W * H * 16)
+    print(f"\n[draw] {W}x{H} sun {sun_length}", flush=True)
+    Renderer(builder).draw(None, a, draw, W, H, color, tr, depth=DeviceBuffer.from_array(depth))
+    synchronize()
+    g_c = color.to_array(np.float32, (H, W, 4))
+    g_t = tr.to_array(np.float32, (H, W, 4))
+    a.close()
+    o_c, o_t = Oracle("f32").render_frame(p, T, S, ivp, draw.camera_position,
+                                           draw.sun_direction, W, H, depth=depth)
+    t_bad = (rel_err(g_t, o_t, 1e-6) > 1e-4).any(-1).mean()
+    c_bad = (rel_err(g_c, o_c, 1e-4) > 1e-3).any(-1).mean()
+    print(f"  pixels outside: transmittance {t_bad:.2e}, radiance {c_bad:.2e}", flush=True)
+    assert t_bad < 1e-3 and c_bad < 1e-3
+    assert np.all(g_c[..., 3] == 0.0) and np.all(g_t[..., 3] == 1.0)
