@@ -691,27 +691,85 @@ __host__ __device__ inline uint32_t hash32(uint32_t x) {
     x ^= x >> 16;
     return x;
 }
+struct RayAttempt {
+    float v1, v2, s;
+};
+__host__ __device__ inline RayAttempt ray_attempt(uint32_t key, uint32_t attempt) {
+    const uint32_t h1 = hash32(key + 2u * attempt), h2 = hash32(key + 2u * attempt + 1u);
+    RayAttempt a;
+    a.v1 = float(h1 >> 8) * (2.0f / 16777216.0f) - 1.0f;
+    a.v2 = float(h2 >> 8) * (2.0f / 16777216.0f) - 1.0f;
+    a.s = a.v1 * a.v1 + a.v2 * a.v2;
+    return a;
+}
+__host__ __device__ inline bool ray_accepted(float s) { return s < 1.0f && s > 0.0f; }
+constexpr uint32_t kRayAttempts = 64;  // then the direction is +z
+// Per frame (block-uniform), then per pixel.
+__host__ __device__ inline uint32_t ray_frame_key(uint64_t seed, uint32_t frame) {
+    return hash32(frame ^ hash32(uint32_t(seed) ^ hash32(uint32_t(seed >> 32))));
+}
+__host__ __device__ inline uint32_t ray_pixel_key(uint32_t frame_key, uint32_t pixel) {
+    return hash32((pixel * 0x9e3779b1u) ^ frame_key);
+}
 __host__ __device__ inline void ray_direction(uint64_t seed, uint32_t frame, uint32_t pixel,
                                               float out[3]) {
-    // Per frame (block-uniform), then per pixel.
-    const uint32_t fk = hash32(frame ^ hash32(uint32_t(seed) ^ hash32(uint32_t(seed >> 32))));
-    const uint32_t key = hash32((pixel * 0x9e3779b1u) ^ fk);
-    for (uint32_t attempt = 0; attempt < 64; ++attempt) {
-        const uint32_t h1 = hash32(key + 2u * attempt), h2 = hash32(key + 2u * attempt + 1u);
-        float v1 = float(h1 >> 8) * (2.0f / 16777216.0f) - 1.0f;
-        float v2 = float(h2 >> 8) * (2.0f / 16777216.0f) - 1.0f;
-        float s = v1 * v1 + v2 * v2;
-        if (s < 1.0f && s > 0.0f) {
-            float q = 2.0f * sqrtf(1.0f - s);
-            out[0] = v1 * q;
-            out[1] = v2 * q;
-            out[2] = 1.0f - 2.0f * s;
+    const uint32_t key = ray_pixel_key(ray_frame_key(seed, frame), pixel);
+    for (uint32_t attempt = 0; attempt < kRayAttempts; ++attempt) {
+        const RayAttempt a = ray_attempt(key, attempt);
+        if (ray_accepted(a.s)) {
+            float q = 2.0f * sqrtf(1.0f - a.s);
+            out[0] = a.v1 * q;
+            out[1] = a.v2 * q;
+            out[2] = 1.0f - 2.0f * a.s;
             return;
         }
     }
     out[0] = 0.0f;
     out[1] = 0.0f;
     out[2] = 1.0f;
+}
+
+// The accepted points of kRayGroup pixels of one thread (pixel0 + i * stride;
+// v1 = v2 = 0 where every attempt failed).  A lane goes to its next pixel as
+// soon as one is done, so a wavefront runs the attempts of its slowest lane's
+// sum over the group (9 for 4 pixels), not the sum of the slowest lanes (14,
+// and 16 as the compiler evaluated four at a time).  Frames are bound by
+// arithmetic, half of it these attempts: 64 x 1920x1080 1248 -> 1128 us (2
+// pixels 1137, 8 1165: registers; 83 VGPRs, held to 72 or 64 1172 and 1257).
+constexpr int kRayGroup = 4;
+__device__ __forceinline__ void ray_points(uint32_t frame_key, uint32_t pixel0, uint32_t stride,
+                                           float (&v1)[kRayGroup], float (&v2)[kRayGroup]) {
+    uint32_t key[kRayGroup];
+#pragma unroll
+    for (int i = 0; i < kRayGroup; ++i) {
+        key[i] = ray_pixel_key(frame_key, pixel0 + uint32_t(i) * stride);
+        v1[i] = v2[i] = 0.0f;
+    }
+    uint32_t k = key[0];
+    int i = 0;
+    uint32_t attempt = 0;
+#pragma unroll 1
+    while (i < kRayGroup) {
+        const RayAttempt a = ray_attempt(k, attempt);
+        const bool ok = ray_accepted(a.s);
+        ++attempt;
+        if (ok || attempt == kRayAttempts) {
+#pragma unroll
+            for (int u = 0; u < kRayGroup; ++u) {
+                v1[u] = ok && i == u ? a.v1 : v1[u];
+                v2[u] = ok && i == u ? a.v2 : v2[u];
+            }
+            ++i;
+            attempt = 0;
+#pragma unroll
+            for (int u = 1; u < kRayGroup; ++u) k = i == u ? key[u] : k;
+        }
+    }
+}
+__device__ __forceinline__ float3 ray_view(float v1, float v2) {
+    const float s = v1 * v1 + v2 * v2;
+    const float q = 2.0f * sqrtf(1.0f - s);
+    return make_float3(v1 * q, v2 * q, 1.0f - 2.0f * s);
 }
 
 // Pixels per thread of the frame kernels (a block shares one slice).
@@ -805,25 +863,32 @@ __device__ void render_frame_block(const DevParams& P, const float4* __restrict_
         sc = slice_consts(P, r);
         __syncthreads();
     }
-    for (int j = 0; j < kFramePixelsPerThread; ++j) {
-        const uint32_t p = pix0 + uint32_t(j) * blockDim.x + threadIdx.x;
-        if (p >= pixels) break;
-        float d[3];
-        ray_direction(seed, frame, p, d);
-        const float3 view = make_float3(d[0], d[1], d[2]);
-        float3 rad, tr;
-        if constexpr (SLICE)
-            sky_radiance_slice(P, sc, s_slice, cam, view, sun, rad, tr);
-        else
-            sky_radiance<H>(P, L, T, S, cam, view, sun, rad, tr);
-        const size_t o = size_t(frame) * pixels + p;  // frame-major output
-        // Written once and not read back by the kernel: non-temporal stores.
-        typedef float v4f __attribute__((ext_vector_type(4)));
-        __builtin_nontemporal_store(v4f{rad.x, rad.y, rad.z, 0.0f},
-                                    reinterpret_cast<v4f*>(rad_out + o));
-        if (trans_out)
-            __builtin_nontemporal_store(v4f{tr.x, tr.y, tr.z, 1.0f},
-                                        reinterpret_cast<v4f*>(trans_out + o));
+    const uint32_t fk = ray_frame_key(seed, frame);
+    static_assert(kFramePixelsPerThread % kRayGroup == 0);
+    for (int g = 0; g < kFramePixelsPerThread; g += kRayGroup) {
+        const uint32_t p0 = pix0 + uint32_t(g) * blockDim.x + threadIdx.x;
+        if (p0 >= pixels) break;
+        float v1[kRayGroup], v2[kRayGroup];
+        ray_points(fk, p0, blockDim.x, v1, v2);
+#pragma unroll
+        for (int j = 0; j < kRayGroup; ++j) {
+            const uint32_t p = p0 + uint32_t(j) * blockDim.x;
+            if (p >= pixels) break;
+            const float3 view = ray_view(v1[j], v2[j]);
+            float3 rad, tr;
+            if constexpr (SLICE)
+                sky_radiance_slice(P, sc, s_slice, cam, view, sun, rad, tr);
+            else
+                sky_radiance<H>(P, L, T, S, cam, view, sun, rad, tr);
+            const size_t o = size_t(frame) * pixels + p;  // frame-major output
+            // Written once and not read back by the kernel: non-temporal stores.
+            typedef float v4f __attribute__((ext_vector_type(4)));
+            __builtin_nontemporal_store(v4f{rad.x, rad.y, rad.z, 0.0f},
+                                        reinterpret_cast<v4f*>(rad_out + o));
+            if (trans_out)
+                __builtin_nontemporal_store(v4f{tr.x, tr.y, tr.z, 1.0f},
+                                            reinterpret_cast<v4f*>(trans_out + o));
+        }
     }
 }
 
