@@ -624,8 +624,13 @@ __global__ __launch_bounds__(256) void k_render_sky_slice(
         fminf(fmaxf(sqrt_nr(d * d + 2.0f * r * mu * d + r * r), L.bottom), L.top);
     const float mu_p = far_away ? d : div_nr(r * mu + d, r_p);
     float4 sc = slice_scattering(C, slice, P.s_nu, P.s_mu, mu, nu, ground);
+    // The far end of an infinite segment, as lut_segment's binary32 gives it:
+    // the length's square plus 2 r mu d is infinite where mu > 0 (the top
+    // boundary), and inf - inf or 0 inf otherwise, a NaN that its clamp turns
+    // into the bottom; the ray leaves it vertically.
+    const float r_d = far_away ? (2.0f * r * mu > 0.0f ? L.top : L.bottom) : r_p;
     const float mu_d = clamp_cosine<float>(mu_p);
-    const float3 far = lut_transmittance(L, T, far_away ? L.top : r_p, ground ? -mu_d : mu_d);
+    const float3 far = lut_transmittance(L, T, r_d, ground ? -mu_d : mu_d);
     const float3 near = slice_transmittance(C, slice + (P.s_nu + 1) * P.s_mu, P.t_mu,
                                             ground ? -mu : mu);
     const float3 tr = lut_ratio(ground ? far : near, ground ? near : far);

@@ -1,7 +1,9 @@
 """Draws large enough for the per-draw LUT slice (1500 x 1001 pixels, which
 fill no block evenly) against the FP32 restatement of render_sky.frag:24-35,
-with and without geometry behind each pixel, and the same draw with a sun
-vector longer than 1, which the slice does not cover.
+with and without geometry behind each pixel, the same draw with a sun vector
+longer than 1, which the slice does not cover, and draws with no geometry at
+all, whose pixels below the horizontal take the far end of an infinite segment
+at the bottom (a NaN of the restatement's binary32, clamped).
 
 Tolerances are those of the small draw's comparison (transmittance 1e-4 at a
 floor of 1e-6 of the maximum, radiance 1e-3 at 1e-4).  One pixel in a thousand
@@ -61,3 +63,45 @@ def test_large_draw_matches_fragment_shader(builder, sun_length):
     print(f"  pixels outside: transmittance {t_bad:.2e}, radiance {c_bad:.2e}", flush=True)
     assert t_bad < 1e-3 and c_bad < 1e-3
     assert np.all(g_c[..., 3] == 0.0) and np.all(g_t[..., 3] == 1.0)
+
+
+def view_along_x(near=0.1):
+    """Inverse of a reverse-Z infinite perspective for a camera 2 km up looking
+    along +x (column-major, [column][row]), in metres."""
+    ivp = np.zeros((4, 4), np.float32)
+    ivp[0] = [0.0, -0.75, 0.0, 0.0]
+    ivp[1] = [0.0, 0.0, -0.5, 0.0]
+    ivp[2] = [0.0, 0.0, 6362e3 / near, 1.0 / near]
+    ivp[3] = [1.0, 0.0, 0.0, 0.0]
+    return ivp
+
+
+# (Even extents: on a centre line the far point at depth 0 is 0/0.)
+@pytest.mark.parametrize("size", [(1500, 1000), (150, 100)], ids=["slice", "direct"])
+def test_draw_without_geometry_matches_fragment_shader(builder, size):
+    w, h = size
+    p = Parameters().replace(**DUMP_SIZES)
+    pa = Atmosphere.build(builder, None, p)
+    pa.wait()
+    a = pa.assert_ready()
+    T = a.download("transmittance").astype(np.float64)
+    S = a.download("scattering").astype(np.float64)
+    ivp = view_along_x()
+    draw = DrawParameters(inverse_viewproj=ivp.tolist(), camera_position=[0.0, 0.0, 6362.0],
+                          sun_direction=[0.6, 0.0, 0.8])
+    color, tr = DeviceBuffer(w * h * 16), DeviceBuffer(w * h * 16)
+    print(f"\n[draw] {w}x{h} without depth", flush=True)
+    Renderer(builder).draw(None, a, draw, w, h, color, tr)
+    synchronize()
+    g_c = color.to_array(np.float32, (h, w, 4))
+    g_t = tr.to_array(np.float32, (h, w, 4))
+    a.close()
+    o_c, o_t = Oracle("f32").render_frame(p, T, S, ivp, draw.camera_position,
+                                           draw.sun_direction, w, h)
+    t_bad = (rel_err(g_t, o_t, 1e-6) > 1e-4).any(-1)
+    c_bad = (rel_err(g_c, o_c, 1e-4) > 1e-3).any(-1)
+    limit = max(1e-3, 1.0 / h)  # the horizon's row (see above)
+    print(f"  pixels outside: transmittance {t_bad.mean():.2e}, radiance {c_bad.mean():.2e}",
+          flush=True)
+    assert np.isfinite(g_c).all() and np.isfinite(g_t).all()
+    assert t_bad.mean() <= limit and c_bad.mean() <= limit
