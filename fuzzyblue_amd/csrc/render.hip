@@ -1012,6 +1012,16 @@ static fb_status end_use(fb_atmosphere* a, hipStream_t s, hipError_t e = hipSucc
     return st;
 }
 
+// Whether work on the stream may become part of a capture.  (The query fails
+// for the legacy stream while a blocking stream is captured.)
+static bool captures(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) == hipSuccess)
+        return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 extern "C" {
 
 fb_status fb_render_sky(fb_builder* b, fb_stream stream, const fb_atmosphere* ac,
@@ -1042,14 +1052,13 @@ fb_status fb_render_sky(fb_builder* b, fb_stream stream, const fb_atmosphere* ac
         (D.cam[0] * D.sun[0] + D.cam[1] * D.sun[1] + D.cam[2] * D.sun[2]) / r;
     // The slice covers what its clamps agree with the per-pixel lookups on: a
     // camera in the atmosphere and a sun vector no longer than 1 (nu of longer
-    // ones leaves the LUT's range).  Where its scratch cannot be had, and in a
-    // captured draw (no allocations there), the draw looks the LUTs up.
+    // ones leaves the LUT's range).  Where its scratch cannot be had, or not
+    // without entering a capture, the draw looks the LUTs up.
     float4* slice = nullptr;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (size_t(width) * height >= fbk::kDrawSliceMinPixels &&
         r >= a->dev.bottom * (1.0f - 1e-6f) && r < a->dev.top * (1.0f - 1e-6f) &&
         D.sun[0] * D.sun[0] + D.sun[1] * D.sun[1] + D.sun[2] * D.sun[2] <= 1.0f + 1e-5f &&
-        hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+        !captures(s) &&
         hipMallocAsync(reinterpret_cast<void**>(&slice), fbk::sky_slice_bytes(a->dev), s) !=
             hipSuccess) {
         (void)hipGetLastError();

@@ -10,6 +10,8 @@ floor of 1e-6 of the maximum, radiance 1e-3 at 1e-4).  One pixel in a thousand
 may exceed them: the horizon, one row of the 1001, is where an ulp of the view
 direction moves a lookup between the two halves of the scattering LUT.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -105,3 +107,37 @@ def test_draw_without_geometry_matches_fragment_shader(builder, size):
           flush=True)
     assert np.isfinite(g_c).all() and np.isfinite(g_t).all()
     assert t_bad.mean() <= limit and c_bad.mean() <= limit
+
+
+def test_large_draw_on_the_legacy_stream_beside_a_captured_one(builder):
+    """While a blocking stream is captured the legacy stream has no capture
+    status and must not allocate: a large draw there goes without the slice."""
+    w, h = 1500, 1000
+    pa = Atmosphere.build(builder, None, Parameters().replace(**DUMP_SIZES))
+    pa.wait()
+    a = pa.assert_ready()
+    paths = {line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line}
+    hip = C.CDLL(paths.pop())
+    draw = DrawParameters(inverse_viewproj=view_along_x().tolist(),
+                          camera_position=[0.0, 0.0, 6362.0], sun_direction=[0.6, 0.0, 0.8])
+    bufs = [DeviceBuffer(w * h * 16) for _ in range(4)]
+    renderer = Renderer(builder)
+    renderer.draw(None, a, draw, w, h, bufs[0], bufs[1])
+    synchronize()
+    s, graph = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(s)) == 0
+    relaxed = 2
+    assert hip.hipStreamBeginCapture(s, relaxed) == 0
+    try:
+        print("\n[draw] legacy stream", flush=True)
+        renderer.draw(None, a, draw, w, h, bufs[2], bufs[3])
+    finally:
+        assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0
+    synchronize()
+    if graph:
+        assert hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamDestroy(s) == 0
+    eager_c, eager_t, c, t = (b.to_array(np.float32, (h, w, 4)) for b in bufs)
+    a.close()
+    assert (rel_err(t, eager_t, 1e-6) > 1e-4).any(-1).mean() < 1e-3
+    assert (rel_err(c, eager_c, 1e-4) > 1e-3).any(-1).mean() < 1e-3
