@@ -19,6 +19,10 @@ LIB = os.path.join(HERE, "libfuzzyblue_hip.so")
 # Micro-kernels measuring the VALU and LDS ceilings (loaded by bench.py only).
 CEILINGS_LIB = os.path.join(HERE, "libfb_ceilings.so")
 CEILINGS_SOURCES = ["ceilings.hip"]
+# The sky lookups' quotients and roots against the IEEE ones (loaded by the
+# tests only).
+CHECKS_LIB = os.path.join(HERE, "libfb_checks.so")
+CHECKS_SOURCES = ["sky_math_check.hip"]
 
 ARCH = os.environ.get("FB_OFFLOAD_ARCH", "gfx950")
 
@@ -74,13 +78,15 @@ def _link(objs, out):
 
 def build(verbose: bool = True) -> str:
     os.makedirs(OUT_DIR, exist_ok=True)
-    srcs = [s for s in SOURCES + CEILINGS_SOURCES if os.path.exists(os.path.join(CSRC, s))]
+    srcs = [s for s in SOURCES + CEILINGS_SOURCES + CHECKS_SOURCES
+            if os.path.exists(os.path.join(CSRC, s))]
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
         objs = dict(zip(srcs, ex.map(_compile, srcs)))
     _link([objs[s] for s in SOURCES], LIB)
     _link([objs[s] for s in CEILINGS_SOURCES], CEILINGS_LIB)
+    _link([objs[s] for s in CHECKS_SOURCES], CHECKS_LIB)
     if verbose:
-        print(f"built {LIB} and {CEILINGS_LIB}")
+        print(f"built {LIB}, {CEILINGS_LIB} and {CHECKS_LIB}")
     return LIB
 
 

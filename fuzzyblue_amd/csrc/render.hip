@@ -7,6 +7,7 @@
 
 #include "atmo_device.hpp"
 #include "runtime.hpp"
+#include "sky_math.hpp"
 
 namespace fbk {
 
@@ -25,40 +26,6 @@ __device__ __forceinline__ float div_rn(float a, float b, float y) {
         d = a / b;
     }
     return d;
-}
-
-// a / b for normal b of ordinary size: a reciprocal refined once, then
-// Markstein's correction -- 9 instruction slots, the compiler's IEEE division
-// about 16.  The refined reciprocal is within an ulp, so the quotient is the
-// IEEE one but for about one pair in 2^23, off by an ulp.
-__device__ __forceinline__ float div_nr(float a, float b) {
-    float y = __builtin_amdgcn_rcpf(b);
-    y = fmaf(fmaf(-b, y, 1.0f), y, y);
-    const float q = a * y;
-    return fmaf(fmaf(-b, q, a), y, q);
-}
-// The same where a wavefront's operands are of ordinary size, else a / b.
-__device__ __forceinline__ float div_any(float a, float b) {
-    float d = div_nr(a, b);
-    if (__builtin_amdgcn_ballot_w64(!(fabsf(b) > 0x1p-100f && fabsf(b) < 0x1p100f &&
-                                      fabsf(a) < 0x1p100f))) {
-        asm volatile("");
-        d = a / b;
-    }
-    return d;
-}
-// sqrt(max(x, 0)) from the hardware's reciprocal square root by two coupled
-// Newton steps, the second with the exact residual: the IEEE root but for
-// rare arguments (an ulp), 13 slots instead of about 20.
-__device__ __forceinline__ float sqrt_nr(float x) {
-    x = fmaxf(x, 0.0f);
-    const float y = __builtin_amdgcn_rsqf(x);
-    float g = x * y, h = 0.5f * y;
-    const float r = fmaf(-h, g, 0.5f);
-    g = fmaf(g, r, g);
-    h = fmaf(h, r, h);
-    g = fmaf(fmaf(-g, g, x), h, g);
-    return x < 0x1p-60f ? __builtin_amdgcn_sqrtf(x) : g;
 }
 
 // The constants of the lookups that depend on the atmosphere and the LUT
@@ -234,10 +201,10 @@ __device__ __forceinline__ float3 extrapolated_single_mie(const SkyLut& L, float
     return make_float3(s.x * q * L.mie_k * L.mie[0], s.y * q * L.mie_k * L.mie[1],
                        s.z * q * L.mie_k * L.mie[2]);
 }
-// util.h:31-34, x^-1.5 by the hardware's reciprocal square root (a few ulp).
+// util.h:31-34
 __device__ __forceinline__ float lut_phase_mie(const SkyLut& L, float nu) {
-    const float y = __builtin_amdgcn_rsqf(L.pm_g1 - L.pm_g2 * nu);
-    return L.pm_k * (1.0f + nu * nu) * (y * y * y);
+    const float x = L.pm_g1 - L.pm_g2 * nu;
+    return div_any(L.pm_k * (1.0f + nu * nu), x * sqrtf(x));
 }
 
 // render_sky.h:21-43 (GLSL mix of the two nu slices).

@@ -1,0 +1,64 @@
+// sky_math.hpp — quotients and square roots of the sky lookups: the bits of
+// the IEEE operations in fewer instructions than the compiler's expansions.
+//
+// They rest on the hardware's v_rcp_f32 and v_rsq_f32 (an ulp): rcp_nr is the
+// correctly rounded reciprocal for every denominator and sqrt_nr the
+// correctly rounded root for every argument, both checked over all binary32
+// values (sky_math_check.hip), and Markstein's correction of a quotient with a
+// correctly rounded reciprocal is the correctly rounded quotient.
+//
+// A wavefront with a lane outside the ranges below takes the compiler's form
+// (a wave-uniform branch; the empty asm statement keeps the compiler from
+// evaluating it unconditionally and selecting), which has the same bits, so a
+// lane's result does not depend on the others'.
+#pragma once
+
+#include "atmo_device.hpp"
+
+namespace fbk {
+
+// 1 / b for 2^-100 < |b| < 2^100.
+__device__ __forceinline__ float rcp_nr(float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    return fmaf(fmaf(-b, y, 1.0f), y, y);
+}
+// a / b for such b and a 0 or of at least 2^-80, where the quotient is normal
+// -- 9 instruction slots, the compiler's division about 16.  (A smaller
+// numerator's quotient may be an ulp off.)
+__device__ __forceinline__ float div_nr(float a, float b) {
+    return div_markstein(a, b, rcp_nr(b));
+}
+// Whether |x| is outside [2^-60, 2^60] (or NaN).
+__device__ __forceinline__ bool extreme(float x) {
+    return __builtin_amdgcn_fmed3f(fabsf(x), 0x1p-60f, 0x1p60f) != fabsf(x);
+}
+// a / b for any operands (but for the sign of a zero quotient).
+__device__ __forceinline__ float div_any(float a, float b) {
+    float d = div_nr(a, b);
+    if (__builtin_amdgcn_ballot_w64(extreme(b) || (extreme(a) && a != 0.0f))) {
+        asm volatile("");
+        d = a / b;
+    }
+    return d;
+}
+// sqrt(max(x, 0)) from the hardware's reciprocal square root by two coupled
+// Newton steps, the second with the exact residual: 15 slots instead of about
+// 20.
+__device__ __forceinline__ float sqrt_nr(float x) {
+    x = fmaxf(x, 0.0f);
+    const float y = __builtin_amdgcn_rsqf(x);
+    float g = x * y, h = 0.5f * y;
+    const float r = fmaf(-h, g, 0.5f);
+    g = fmaf(g, r, g);
+    h = fmaf(h, r, h);
+    g = fmaf(fmaf(-g, g, x), h, g);
+    // 2^-60 <= x < 2^126 by the bits.
+    const bool inside = __float_as_uint(x) - 0x21800000u < 0x7e800000u - 0x21800000u;
+    if (__builtin_amdgcn_ballot_w64(!inside && x != 0.0f)) {
+        asm volatile("");
+        g = sqrtf(x);
+    }
+    return x == 0.0f ? 0.0f : g;
+}
+
+}  // namespace fbk
