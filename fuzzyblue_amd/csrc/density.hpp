@@ -81,16 +81,6 @@ __device__ __forceinline__ float3 prof_lerp_i(const ProfEntry* __restrict__ prof
     float2 b = e->b;
     return make_float3(fmaf(a.w, f, a.x), fmaf(b.x, f, a.y), fmaf(b.y, f, a.z));
 }
-// The same over entries that hold each cell's line as its value at x = 0 and
-// its slope: one instruction fewer per lookup (no fract), 5% of an order >= 3
-// launch (double 2.54 -> 2.41 ms).  The value at 0 is rounded at up to NU + 1
-// slopes' size, as x itself is; the LUTs' errors against 64 bits stay the same.
-__device__ __forceinline__ float3 prof_line(const ProfEntry* __restrict__ prof, float x) {
-    const ProfEntry* e = prof + int(x);
-    const float4 a = e->a;
-    const float2 b = e->b;
-    return make_float3(fmaf(a.w, x, a.x), fmaf(b.x, x, a.y), fmaf(b.y, x, a.z));
-}
 // The same for a Rayleigh / Mie pair of profiles.
 __device__ __forceinline__ void pair_lerp_i(const PairEntry* __restrict__ prof, float e1,
                                             float3& R, float3& M) {
@@ -150,7 +140,7 @@ __device__ __forceinline__ void density_row(const DenConst& k, const DenTexel* d
                 S = make_float3(fmaf(qb, B.x, qa * A.x), fmaf(qb, B.y, qa * A.y),
                                 fmaf(qb, B.z, qa * A.z));
             } else {
-                const float3 A = prof_line(row.pr, ca), B = prof_line(row.pr, cb);
+                const float3 A = prof_lerp_i(row.pr, ca), B = prof_lerp_i(row.pr, cb);
                 S = make_float3(A.x + B.x, A.y + B.y, A.z + B.z);
             }
             a[u].x = fmaf(p.x, S.x, a[u].x);
@@ -403,8 +393,8 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
     const int many_mask = __builtin_amdgcn_readfirstlane(s_masks[2]);
     // 2. Entries.  Order 1 (single scattering): (value, delta) times the phase
     // constants, rayleigh x 3/(16 pi), mie x 3/(8 pi)(1-g^2)/(2+g^2) (util.h:
-    // 26-34).  Later orders: each cell's line (prof_line), the affine part of
-    // the ground term included.
+    // 26-34).  Later orders: (value, delta), the affine part of the ground term
+    // included.
     for (int e = tid; e < kDenTheta * nent; e += blockDim.x) {
         const int row = e / nent, k = e % nent;  // entry k holds slot k-1
         const float4 v = s_raw[row * nslots + k], w = s_raw[row * nslots + k + 1];
@@ -422,11 +412,9 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
             const float dn = fmaf(float(k) - kc.hnu1, h, -c_den_cos[row] * osz);  // nu1 - centre
             const float3 d = make_float3(fmaf(gs.x, h, w.x - v.x), fmaf(gs.y, h, w.y - v.y),
                                          fmaf(gs.z, h, w.z - v.z));
-            const float kf = -float(k);
             ProfEntry p;
-            p.a = make_float4(fmaf(kf, d.x, v.x + fmaf(gs.x, dn, gl.x)),
-                              fmaf(kf, d.y, v.y + fmaf(gs.y, dn, gl.y)),
-                              fmaf(kf, d.z, v.z + fmaf(gs.z, dn, gl.z)), d.x);
+            p.a = make_float4(v.x + fmaf(gs.x, dn, gl.x), v.y + fmaf(gs.y, dn, gl.y),
+                              v.z + fmaf(gs.z, dn, gl.z), d.x);
             p.b = make_float2(d.y, d.z);
             p.pad = make_float2(0.0f, 0.0f);
             s_prof[e] = p;
@@ -474,7 +462,7 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
                                 fmaf(q, L.y, fmaf(gs.y, dn, gl.y)),
                                 fmaf(q, L.z, fmaf(gs.z, dn, gl.z)));
             } else {
-                L = prof_line(row.pr, fmaf(dn, kc.hnu, row.c));
+                L = prof_lerp_i(row.pr, fmaf(dn, kc.hnu, row.c));
             }
             if ((kink_mask >> l) & 1) {
                 const float4 k = s_kink[l];
