@@ -191,15 +191,17 @@ __device__ __forceinline__ float4 lut_scattering(const SkyLut& L, const float4* 
                        a0.z * (1.0f - lerp) + a1.z * lerp, a0.w * (1.0f - lerp) + a1.w * lerp);
 }
 
-// render_sky.h:9-19, the red channel (s.x * s.w / s.x * k * ratio) and all.
-__device__ __forceinline__ float single_mie_red(const SkyLut& L, float4 s) {
-    return s.x <= 0.0f ? 0.0f : div_any(s.x * s.w, s.x) * L.mie_k * L.mie[0];
-}
+// render_sky.h:9-19, all channels and the red one.  Products before quotients,
+// as there: GetSkyRadianceToPoint takes differences of nearly equal values, in
+// which another rounding shows.
 __device__ __forceinline__ float3 extrapolated_single_mie(const SkyLut& L, float4 s) {
     if (s.x <= 0.0f) return make_float3(0.0f, 0.0f, 0.0f);
-    const float q = div_any(s.w, s.x);
-    return make_float3(s.x * q * L.mie_k * L.mie[0], s.y * q * L.mie_k * L.mie[1],
-                       s.z * q * L.mie_k * L.mie[2]);
+    const float3 q = scale_div_any(make_float3(s.x, s.y, s.z), s.w, s.x);
+    return make_float3(q.x * L.mie_k * L.mie[0], q.y * L.mie_k * L.mie[1],
+                       q.z * L.mie_k * L.mie[2]);
+}
+__device__ __forceinline__ float single_mie_red(const SkyLut& L, float4 s) {
+    return s.x <= 0.0f ? 0.0f : div_any(s.x * s.w, s.x) * L.mie_k * L.mie[0];
 }
 // util.h:31-34
 __device__ __forceinline__ float lut_phase_mie(const SkyLut& L, float nu) {

@@ -28,16 +28,35 @@ __device__ __forceinline__ float rcp_nr(float b) {
 __device__ __forceinline__ float div_nr(float a, float b) {
     return div_markstein(a, b, rcp_nr(b));
 }
-// Whether |x| is outside [2^-60, 2^60] (or NaN).
-__device__ __forceinline__ bool extreme(float x) {
-    return __builtin_amdgcn_fmed3f(fabsf(x), 0x1p-60f, 0x1p60f) != fabsf(x);
+// Whether |x| is outside [lo, hi] (or NaN).
+__device__ __forceinline__ bool outside(float x, float lo, float hi) {
+    return __builtin_amdgcn_fmed3f(fabsf(x), lo, hi) != fabsf(x);
 }
+// Denominators and numerators (other than 0) that div_nr divides exactly in
+// any combination.
+__device__ __forceinline__ bool extreme_den(float b) { return outside(b, 0x1p-60f, 0x1p40f); }
+__device__ __forceinline__ bool extreme_num(float a) { return outside(a, 0x1p-80f, 0x1p60f); }
 // a / b for any operands (but for the sign of a zero quotient).
 __device__ __forceinline__ float div_any(float a, float b) {
     float d = div_nr(a, b);
-    if (__builtin_amdgcn_ballot_w64(extreme(b) || (extreme(a) && a != 0.0f))) {
+    if (__builtin_amdgcn_ballot_w64(extreme_den(b) || (extreme_num(a) && a != 0.0f))) {
         asm volatile("");
         d = a / b;
+    }
+    return d;
+}
+// (s a) / b per channel, by one reciprocal.
+__device__ __forceinline__ float3 scale_div_any(float3 a, float s, float b) {
+    const float3 n = make_float3(a.x * s, a.y * s, a.z * s);
+    const float y = rcp_nr(b);
+    float3 d = make_float3(div_markstein(n.x, b, y), div_markstein(n.y, b, y),
+                           div_markstein(n.z, b, y));
+    const float lo = fminf(fminf(fabsf(n.x), fabsf(n.y)), fabsf(n.z)),
+                hi = fmaxf(fmaxf(fabsf(n.x), fabsf(n.y)), fabsf(n.z));
+    if (__builtin_amdgcn_ballot_w64(extreme_den(b) ||
+                                    ((lo < 0x1p-80f || hi > 0x1p60f) && s != 0.0f))) {
+        asm volatile("");
+        d = make_float3(n.x / b, n.y / b, n.z / b);
     }
     return d;
 }

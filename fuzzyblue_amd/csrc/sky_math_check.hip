@@ -40,14 +40,19 @@ __global__ __launch_bounds__(kThreads) void k_reciprocals(Found* f) {
         note(f, in && differs(fbk::rcp_nr(b), 1.0f / b), b, 0.0f);
     }
 }
-// any: div_any on all pairs, else div_nr where its ranges hold.
+// kind 0: div_nr where its ranges hold, 1: div_any, 2: scale_div_any (b / 3 as
+// the scale).
 __global__ __launch_bounds__(kThreads) void k_quotients(const float* a, const float* b, size_t n,
-                                                        bool any, Found* f) {
+                                                        int kind, Found* f) {
     const size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x;
     const float x = i < n ? a[i] : 1.0f, y = i < n ? b[i] : 1.0f, want = x / y;
     bool bad;
-    if (any) {
+    if (kind == 1) {
         bad = differs(fbk::div_any(x, y), want);
+    } else if (kind == 2) {
+        const float s = y / 3.0f;
+        const float3 d = fbk::scale_div_any(make_float3(x, x * 0.375f, 1.0f), s, y);
+        bad = differs(d.x, x * s / y) || differs(d.y, x * 0.375f * s / y) || differs(d.z, s / y);
     } else {
         const bool in = fabsf(y) > 0x1p-100f && fabsf(y) < 0x1p100f && fabsf(x) >= 0x1p-80f &&
                         fabsf(x) < 0x1p100f && fabsf(want) >= 0x1p-126f && fabsf(want) < 0x1p127f;
@@ -85,10 +90,10 @@ int fbc_reciprocal(unsigned long long* count, float example[2]) {
     return run(count, example, [](Found* f) { k_reciprocals<<<kBlocks, kThreads>>>(f); });
 }
 // a, b: n values each in device memory.
-int fbc_quotient(const float* a, const float* b, size_t n, int any, unsigned long long* count,
+int fbc_quotient(const float* a, const float* b, size_t n, int kind, unsigned long long* count,
                  float example[2]) {
     return run(count, example, [=](Found* f) {
-        k_quotients<<<unsigned((n + kThreads - 1) / kThreads), kThreads>>>(a, b, n, any != 0, f);
+        k_quotients<<<unsigned((n + kThreads - 1) / kThreads), kThreads>>>(a, b, n, kind, f);
     });
 }
 

@@ -21,10 +21,10 @@ def call(fn, *args):
     return count.value, [x.hex() for x in example]
 
 
-def quotients(a, b, any_operands):
+def quotients(a, b, kind):
     a, b = (np.ascontiguousarray(x, np.float32) for x in (a, b))
     da, db = DeviceBuffer.from_array(a), DeviceBuffer.from_array(b)
-    return call("fbc_quotient", da.ptr, db.ptr, C.c_size_t(a.size), C.c_int(any_operands))
+    return call("fbc_quotient", da.ptr, db.ptr, C.c_size_t(a.size), C.c_int(kind))
 
 
 @pytest.mark.parametrize("fn", ["fbc_sqrt", "fbc_reciprocal"])
@@ -43,13 +43,13 @@ def boundary_values():
     return np.concatenate([v, -v])
 
 
-@pytest.mark.parametrize("any_operands", [0, 1])
-def test_quotients_of_boundary_values(builder, any_operands):
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_quotients_of_boundary_values(builder, kind):
     v = boundary_values()
     a, b = np.repeat(v, v.size), np.tile(v, v.size)
     # Each pair with a wavefront of its own, then all mixed.
     for x, y in ((np.repeat(a, 64), np.repeat(b, 64)), (a, b)):
-        count, example = quotients(x, y, any_operands)
+        count, example = quotients(x, y, kind)
         assert count == 0, example
 
 
@@ -58,13 +58,13 @@ def random_values(rng, n, lo, hi):
     return (x * np.where(rng.random(n) < 0.5, -1, 1)).astype(np.float32)
 
 
-@pytest.mark.parametrize("any_operands", [0, 1])
-def test_quotients_of_random_pairs(builder, any_operands):
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_quotients_of_random_pairs(builder, kind):
     rng = np.random.default_rng(11)
     n = 1 << 22
     for lo, hi in ((-2, 2), (-60, 60), (-80, 46)):
         count, example = quotients(random_values(rng, n, lo, hi), random_values(rng, n, lo, hi),
-                                   any_operands)
+                                   kind)
         assert count == 0, example
 
 
@@ -74,5 +74,6 @@ def test_quotients_beside_an_extreme_lane(builder):
     a, b = random_values(rng, n, -20, 20), random_values(rng, n, -20, 20)
     a[::64] = random_values(rng, n // 64, -126, -90)
     b[32::128] = np.inf
-    count, example = quotients(a, b, 1)
-    assert count == 0, example
+    for kind in (1, 2):
+        count, example = quotients(a, b, kind)
+        assert count == 0, example
