@@ -30,12 +30,13 @@ static __constant__ float4 c_den_dir[kDenTheta * kDenPhi];  // (cos phi sin t, s
 static __constant__ float c_den_cos[kDenTheta];
 static __constant__ float c_den_sin[kDenTheta];
 static __constant__ float2 c_den_phi[kDenPhi / 2];  // cos phi, sin phi of the half turn m < 16
+static __constant__ float c_den_cx[kDenTheta * kDenPhi / 2];  // c_den_dir's x of the half turn
 static __constant__ double c_den_cos_d[kDenTheta];
 
 static hipError_t upload_density_tables() {
     float4 den[kDenTheta * kDenPhi];
     float2 phis[kDenPhi / 2];
-    float dcos[kDenTheta], dsin[kDenTheta];
+    float dcos[kDenTheta], dsin[kDenTheta], cx[kDenTheta * kDenPhi / 2];
     double dcos_d[kDenTheta];
     const float PI = 3.14159265358979323846f;
     const float dphi = PI / float(16), dtheta = PI / float(16);
@@ -51,6 +52,7 @@ static hipError_t upload_density_tables() {
             if (m < kDenPhi / 2) phis[m] = make_float2(cosf(phi), sinf(phi));
             float domega = dtheta * dphi * sinf(theta);
             den[l * kDenPhi + m] = make_float4(cosf(phi) * st, sinf(phi) * st, ct, domega);
+            if (m < kDenPhi / 2) cx[l * kDenPhi / 2 + m] = den[l * kDenPhi + m].x;
         }
     }
     hipError_t e;
@@ -58,6 +60,7 @@ static hipError_t upload_density_tables() {
     if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_cos), dcos, sizeof(dcos))) != hipSuccess) return e;
     if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_sin), dsin, sizeof(dsin))) != hipSuccess) return e;
     if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_phi), phis, sizeof(phis))) != hipSuccess) return e;
+    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_cx), cx, sizeof(cx))) != hipSuccess) return e;
     return hipMemcpyToSymbol(HIP_SYMBOL(c_den_cos_d), dcos_d, sizeof(dcos_d));
 }
 
