@@ -105,6 +105,7 @@ FB_PASS_SCATTERING_DENSITY = 4
 FB_PASS_INDIRECT_IRRADIANCE = 5
 FB_PASS_MULTIPLE_SCATTERING = 6
 FB_PASS_GEOMETRY = 7
+FB_XCD_REMAP_DEFAULT = 1 << FB_PASS_MULTIPLE_SCATTERING
 
 FB_PASS_NAMES = {
     0: "transmittance",

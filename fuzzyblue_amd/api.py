@@ -124,7 +124,7 @@ class Builder:
 
     def set_tuning(self, params: Parameters, **sizes):
         """Install block sizes (fb_tuning field names; omitted = default)."""
-        t = abi.fb_tuning()
+        t = abi.fb_tuning(xcd_remap=abi.FB_XCD_REMAP_DEFAULT)
         for k, v in sizes.items():
             if k == "best_ms" or not hasattr(t, k):
                 raise AttributeError(k)

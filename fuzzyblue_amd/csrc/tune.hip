@@ -18,6 +18,8 @@
 
 namespace fbrt {
 
+static_assert(FB_XCD_REMAP_DEFAULT == fbk::Tuning{}.remap, "default block order mirror");
+
 TuneKey tune_key(const fb_parameters& p) {
     return TuneKey{p.flags & (FB_FLAG_PRECISE | FB_FLAG_F16_STORAGE), p.transmittance_mu_size, p.transmittance_r_size,
                    p.scattering_r_size,       p.scattering_mu_size,    p.scattering_mu_s_size,

@@ -201,8 +201,8 @@ fb_status fb_pending_relaunch(fb_pending_atmosphere *pa, fb_stream stream);
  * choice gives bit-identical LUTs; builds (plain and batched) started
  * after the tuning is set use it. */
 typedef struct fb_tuning {
-    uint32_t single_scattering_threads;   /* 64, 128 or 256 per (r, mu) row */
-    uint32_t density_order2_threads;      /* 64, 128 or 256 per (r, mu_s) tile */
+    uint32_t single_scattering_threads;   /* 64, 128, 192 or 256 per (r, mu) row */
+    uint32_t density_order2_threads;      /* the same per (r, mu_s) tile */
     uint32_t density_threads;             /* the same for orders >= 3 */
     uint32_t indirect_order1_waves;       /* 1, 2 or 4 wavefronts per block */
     uint32_t indirect_waves;              /* the same for orders >= 2 */
@@ -213,11 +213,13 @@ typedef struct fb_tuning {
     uint32_t xcd_remap; /* bit p set (p = FB_PASS_SINGLE_SCATTERING,
                            FB_PASS_SCATTERING_DENSITY or
                            FB_PASS_MULTIPLE_SCATTERING): that pass gives each
-                           of the 8 XCDs a contiguous share of its blocks
-                           (untuned classes: multiple scattering only) */
+                           of the 8 XCDs a contiguous share of its blocks.
+                           0 is none, not the default: that is
+                           FB_XCD_REMAP_DEFAULT, which untuned classes use */
     float best_ms[6]; /* fb_builder_autotune: measured ms per launch of each
                          chosen shape, in field order; 0 otherwise */
 } fb_tuning;
+#define FB_XCD_REMAP_DEFAULT (1u << 6) /* multiple scattering only */
 
 /* Time every candidate block size of each tunable pass on a scratch LUT
  * set of p's sizes (enqueued on `stream`, synchronised), keep the fastest
@@ -228,8 +230,9 @@ fb_status fb_builder_autotune(fb_builder *b, fb_stream stream,
  * defaults in *out) when the class was never tuned. */
 fb_status fb_builder_get_tuning(fb_builder *b, const fb_parameters *p,
                                 fb_tuning *out);
-/* Install block sizes (0 = default) for p's size class, e.g. a table
- * saved from an earlier autotune; FB_EINVAL if one is not valid there. */
+/* Install block sizes (0 = default) and the block order (as given) for p's
+ * size class, e.g. a table saved from an earlier autotune; FB_EINVAL if one
+ * is not valid there. */
 fb_status fb_builder_set_tuning(fb_builder *b, const fb_parameters *p,
                                 const fb_tuning *t);
 

@@ -91,3 +91,16 @@ def test_batch_uses_tuning_and_matches_plain():
     for pa in pend:
         pa.close()
     b.close()
+
+
+def test_omitted_block_order_is_the_default():
+    b = Builder(0)
+    p = Parameters().replace(**DUMP_SIZES)
+    _, untuned = b.tuning(p)
+    b.set_tuning(p, density_threads=128)
+    tuned, t = b.tuning(p)
+    assert tuned and t["density_threads"] == 128
+    assert t["xcd_remap"] == untuned["xcd_remap"] == abi.FB_XCD_REMAP_DEFAULT
+    b.set_tuning(p, xcd_remap=0)
+    assert b.tuning(p)[1]["xcd_remap"] == 0
+    b.close()
