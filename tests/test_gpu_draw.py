@@ -15,7 +15,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from fuzzyblue_amd import (Atmosphere, DeviceBuffer, DrawParameters, Parameters, Renderer,
+from fuzzyblue_amd import (Atmosphere, DeviceBuffer, DrawParameters, Parameters, Renderer, abi,
                            synchronize)
 from fuzzyblue_amd.params import DUMP_SIZES
 from oracle import Oracle
@@ -141,3 +141,45 @@ def test_large_draw_on_the_legacy_stream_beside_a_captured_one(builder):
     a.close()
     assert (rel_err(t, eager_t, 1e-6) > 1e-4).any(-1).mean() < 1e-3
     assert (rel_err(c, eager_c, 1e-4) > 1e-3).any(-1).mean() < 1e-3
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["binary32", "binary16"])
+@pytest.mark.parametrize("form", ["composite", "composite_no_transmittance", "no_transmittance"])
+def test_large_draw_forms_match_fragment_shader(builder, f16, form):
+    """The slice draw's other outputs (composited over a background, without a
+    transmittance image), on both storage types."""
+    w, h = 1500, 1000
+    p = Parameters().replace(**DUMP_SIZES, flags=abi.FB_FLAG_F16_STORAGE if f16 else 0)
+    pa = Atmosphere.build(builder, None, p)
+    pa.wait()
+    a = pa.assert_ready()
+    T = a.download("transmittance").astype(np.float64)
+    S = a.download("scattering").astype(np.float64)
+    near = 0.1
+    ivp = view_along_x(near)
+    draw = DrawParameters(inverse_viewproj=ivp.tolist(), camera_position=[0.0, 0.0, 6362.0],
+                          sun_direction=[0.6, 0.0, 0.8])
+    rng = np.random.default_rng(5)
+    depth = rng.uniform(near / 50e3, near / 500.0, (h, w)).astype(np.float32)
+    depth[: h // 2] = 0.0
+    back = rng.uniform(0.0, 0.2, (h, w, 4)).astype(np.float32)
+    color = DeviceBuffer.from_array(back)
+    tr = None if "no_transmittance" in form else DeviceBuffer(w * h * 16)
+    print(f"\n[draw] {w}x{h} {form} binary{16 if f16 else 32}", flush=True)
+    Renderer(builder).draw(None, a, draw, w, h, color, tr,
+                           depth=DeviceBuffer.from_array(depth), composite="composite" in form)
+    synchronize()
+    g_c = color.to_array(np.float32, (h, w, 4))
+    a.close()
+    o_c, o_t = Oracle("f32").render_frame(p, T, S, ivp, draw.camera_position,
+                                           draw.sun_direction, w, h, depth=depth)
+    want = np.asarray(o_c, np.float64)
+    if "composite" in form:
+        want = want + back * np.asarray(o_t, np.float64)
+        assert np.array_equal(g_c[..., 3], back[..., 3])
+    else:
+        assert np.all(g_c[..., 3] == 0.0)
+    assert (rel_err(g_c, want, 1e-4) > 1e-3).any(-1).mean() < 1e-3
+    if tr is not None:
+        g_t = tr.to_array(np.float32, (h, w, 4))
+        assert (rel_err(g_t, o_t, 1e-6) > 1e-4).any(-1).mean() < 1e-3

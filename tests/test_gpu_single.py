@@ -4,6 +4,9 @@ different paths, on the GPU's own transmittance against the FP64 oracle's pass
 block evenly, transmittance rows of up to two columns per thread (loaded ahead)
 and wider ones, and a row too narrow for staging.
 
+FP32 mode, whose quotients by the sample tables' denominators are Markstein's,
+against the FP32 restatement on the same cases.
+
 Tolerance 1e-4 (floor 1e-6 x the maximum), the bar of the
 pass-by-pass comparisons.
 """
@@ -48,3 +51,30 @@ def test_single_paths_vs_oracle(name):
         err = np.abs(x - want) / np.maximum(np.abs(want), 1e-6 * np.abs(want).max())
         print(f"  max {err.max():.2e}", flush=True)
         assert err.max() < 1e-4
+
+
+# Both sides evaluate the same binary32 operations, so what remains is the
+# order of the 51 samples' sums and the transmittance taps' interpolation: up
+# to 51 roundings of 2^-24, 3e-6.
+@pytest.mark.parametrize("name", CASES)
+def test_single_paths_vs_restatement(name):
+    (r, mu, mus, nu), tmu, threads = CASES[name]
+    p = Parameters().replace(scattering_r_size=r, scattering_mu_size=mu,
+                             scattering_mu_s_size=mus, scattering_nu_size=nu,
+                             transmittance_mu_size=tmu, transmittance_r_size=17, order=1)
+    b = Builder(0)
+    b.set_tuning(p, single_scattering_threads=threads)
+    print(f"\n[single] fp32 {name} {p.scattering_extent()}", flush=True)
+    pa = Atmosphere.build(b, None, p)
+    pa.wait()
+    got = [pa.download_scratch("delta_rayleigh"), pa.download_scratch("delta_mie"),
+           pa.atmosphere().download("scattering")]
+    T = pa.atmosphere().download("transmittance")
+    pa.close()
+    b.close()
+    for g, want in zip(got, Oracle("f32").pass_single_scattering(p, T)):
+        want = np.asarray(want, np.float64).reshape(-1, 4)[:, :3]
+        x = g.reshape(-1, 4)[:, :3].astype(np.float64)
+        err = np.abs(x - want) / np.maximum(np.abs(want), 1e-6 * np.abs(want).max())
+        print(f"  max {err.max():.2e}", flush=True)
+        assert err.max() < 3e-6
