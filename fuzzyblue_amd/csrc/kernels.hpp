@@ -133,16 +133,16 @@ struct DenLayout {
     }
 };
 // Density texels per thread.  The texels of one mu share nu2 = omega.omega_i
-// and the phase weight of every direction pair (13 of a lone texel's 34
+// and the phase weight of every direction pair (13 of a lone texel's 36
 // instruction slots per pair), so a thread takes as many as divide the inner
 // nu indices evenly: 7, 6, 4 or 2, while the set's tiles fill at least
 // kDenMinWaves wavefronts (4 per SIMD; below that, occupancy is worth more
 // than the shared work).  Order >= 3 and order 2, ms per launch: double (14
-// inner) 7: 2.22 / 4.70, 4: 2.36 / 4.99 (2 of 16 places idle), 2: 2.42 / 5.11;
-// default (6 inner) 6: 0.168 / 0.325, 2: 0.174 / 0.348; default in FP32 mode
-// (8) 4: 0.181 / 0.385, 2: 0.189 / 0.408; 27x64x26x18 (16 inner, 3,510 waves
-// at 4) 4: 0.221 / 0.470, 2: 0.142 / 0.305.  A texel's own operations and
-// their order do not depend on it.
+// inner) 7: 2.08 / 4.35, 2: 2.50 / 4.93; default (6 inner) 6: 0.186 / 0.321,
+// 2: 0.188 / 0.352; default in FP32 mode (8) 4: 0.173 / 0.347, 2: 0.180 /
+// 0.354; 27x64x26x18 (16 inner, 3,510 waves at 4) 4: 0.248 / 0.465, 2: 0.154 /
+// 0.305.  (5, and 3 with its few shared texels, have no kernel.)  A texel's own
+// operations and their order do not depend on it.
 constexpr int kDenMinWaves = 4096;
 constexpr int kDenPairMinTexels = 512;  // tiles of fewer texels keep one per thread
 __host__ __device__ inline int den_tpx(const DevParams& P) {
@@ -154,13 +154,14 @@ __host__ __device__ inline int den_tpx(const DevParams& P) {
             return t;
     return inner % 2 == 0 && P.s_mu * P.s_nu >= kDenPairMinTexels ? 2 : 1;
 }
-// Blocks of 256 threads per CU the density kernels are compiled for.  One
-// texel per thread: 4 (8 blocks, 64 VGPRs, spill: 0.066 instead of 0.041 ms
-// per order >= 3 launch of a half-resolution set, whose blocks do not fill
-// the chip).  Two: 7 at order >= 3, 5 at order 2 (at double 2.54 ms, 6 2.54,
-// 8 2.60; order 2 with 6 5.30 instead of 5.23).
+// Blocks of 256 threads per CU the density kernels are compiled for; order >= 3
+// and order 2, ms per launch.  One texel per thread: 4 (8 blocks spill: half
+// resolution 0.045 / 0.081 instead of 0.041 / 0.063).  Two: 7 and 5
+// (27x64x26x18 0.154 / 0.305, one more 0.164 / 0.308, one less 0.165 / 0.296).
+// Four and six: 4 (default 0.186 / 0.321, with 5 0.213 / 0.343, 3 0.193 /
+// 0.399).  Seven: 4 (double 2.08 / 4.35, with 3 2.48 / 4.64).
 __host__ __device__ constexpr int den_occupancy(int tpx, bool single) {
-    return tpx == 2 ? (single ? 5 : 7) : tpx == 7 ? 3 : 4;
+    return tpx == 2 ? (single ? 5 : 7) : 4;
 }
 constexpr int kSsMaxStagedMu = 2048;
 // Multiple scattering over rows of at most kMsChunkMaxW texels (small LUT
