@@ -242,13 +242,13 @@ __device__ __forceinline__ void density_ground(const DenConst& k, const DenTexel
 // a thread only weighs it with its mu's phases: at azimuth 0 the value of
 // direction m, at azimuth pi that of 15 - m.
 //
-// Bound by instruction issue (about 24 VALU slots per direction pair and
-// inner texel at seven texels per thread, 31 at one, 10 per outer texel; 0.6
+// Bound by instruction issue (about 26 VALU slots per direction pair and
+// inner texel at seven texels per thread, 33 at one, 10 per outer texel; 0.6
 // of the 2.4 GHz issue peak at double).  ms per order >= 3 launch / order 2,
 // with a ground lookup per direction on ground rows, every texel on the
-// general path and two texels per thread before: default 0.236 -> 0.168 /
-// 0.393 -> 0.325, double 3.48 -> 2.22 / 6.11 -> 4.65, half resolution 0.066 ->
-// 0.040 / 0.085 -> 0.062.
+// general path and two texels per thread before: default 0.236 -> 0.186 /
+// 0.393 -> 0.321, double 3.48 -> 2.08 / 6.11 -> 4.35, half resolution 0.066 ->
+// 0.041 / 0.085 -> 0.063.
 template <typename G, bool SINGLE, bool H, int TPX = 1>
 __device__ __forceinline__ void scattering_density_block(const DevParams& P, const int bx, const int by, const int bz, const float4* __restrict__ DG, const float4* __restrict__ dR,
     const float4* __restrict__ dM, const float4* __restrict__ dMS, const float4* __restrict__ dE,

@@ -159,7 +159,8 @@ __host__ __device__ inline int den_tpx(const DevParams& P) {
 // resolution 0.045 / 0.081 instead of 0.041 / 0.063).  Two: 7 and 5
 // (27x64x26x18 0.154 / 0.305, one more 0.164 / 0.308, one less 0.165 / 0.296).
 // Four and six: 4 (default 0.186 / 0.321, with 5 0.213 / 0.343, 3 0.193 /
-// 0.399).  Seven: 4 (double 2.08 / 4.35, with 3 2.48 / 4.64).
+// 0.399).  Seven: 4, with 12 to 32 registers spilled (double 2.08 / 4.35, with
+// 3 and none spilled 2.48 / 4.64).
 __host__ __device__ constexpr int den_occupancy(int tpx, bool single) {
     return tpx == 2 ? (single ? 5 : 7) : 4;
 }

@@ -1739,9 +1739,9 @@ unsigned default_threads(const DevParams& P, int pass, int order) {
         case kPassMultiple:  // one texel per thread
             return std::min(unsigned(kMsMaxThreads), row);
         case kPassDensity:  // 256, or the tile's threads (in 256-thread blocks, half of them
-                            // idle, a 64x64x32x8 FP32 launch took 0.201 ms, not 0.164; a
+                            // idle, a 64x64x32x8 FP32 launch takes 0.235 ms, not 0.176; a
                             // larger tile cut evenly, 3 x 192 for 256 + 256 + 64, is slower:
-                            // 0.158 instead of 0.142 ms at 27x64x26x18)
+                            // 0.171 instead of 0.154 ms at 27x64x26x18)
             return std::min(256u, cdiv(unsigned(DenLayout(P, den_tpx(P)).total), 64) * 64);
         case kPassIndirect: {
             const size_t per_wave = indirect_lds_bytes_per_wave(P.s_nu, (order - 1) == 1);

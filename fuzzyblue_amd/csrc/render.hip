@@ -211,7 +211,7 @@ __device__ __forceinline__ float lut_phase_mie(const SkyLut& L, float nu) {
 
 // render_sky.h:21-43 (GLSL mix of the two nu slices).
 template <bool H>
-__device__ __forceinline__ float4 combined_scattering(const DevParams& P, const SkyLut& L,
+__device__ __forceinline__ float4 combined_scattering(const SkyLut& L,
                                                       const float4* __restrict__ S, float r,
                                                       float mu, float mu_s, float nu, bool ground,
                                                       float3& mie) {
@@ -249,7 +249,7 @@ __device__ void sky_radiance(const DevParams& P, const SkyLut& L, const float4* 
     float3 mie;
     float4 sc;
     if (!SHADOW || shadow_length == 0.0f) {
-        sc = combined_scattering<H>(P, L, S, r, mu, mu_s, nu, ground, mie);
+        sc = combined_scattering<H>(L, S, r, mu, mu_s, nu, ground, mie);
     } else {
         // Eq. (18): the scattering seen from x + l v, attenuated by
         // T(x, x + l v) (render_sky.h:86-105).
@@ -257,7 +257,7 @@ __device__ void sky_radiance(const DevParams& P, const SkyLut& L, const float4* 
         const float r_p = clamp_radius<float>(P, sqrtf(d * d + 2.0f * r * mu * d + r * r));
         const float mu_p = (r * mu + d) / r_p;
         const float mu_s_p = (r * mu_s + d * nu) / r_p;
-        sc = combined_scattering<H>(P, L, S, r_p, mu_p, mu_s_p, nu, ground, mie);
+        sc = combined_scattering<H>(L, S, r_p, mu_p, mu_s_p, nu, ground, mie);
         const float3 st = lut_segment(L, T, r, mu, shadow_length, ground);
         sc = make_float4(sc.x * st.x, sc.y * st.y, sc.z * st.z, sc.w);
         mie = make_float3(mie.x * st.x, mie.y * st.y, mie.z * st.z);
@@ -270,9 +270,9 @@ __device__ void sky_radiance(const DevParams& P, const SkyLut& L, const float4* 
 // (:158-160, :172-177) when SHADOW and shadow_length > 0.
 template <bool H, bool SHADOW = false>
 __device__ void sky_radiance_to_point(const DevParams& P, const SkyLut& L,
-                                      const float4* __restrict__ T, const float4* __restrict__ S, float3 camera, float3 view,
-                                      float3 point, float3 sun, float3& rad, float3& trans,
-                                      float shadow_length = 0.0f) {
+                                      const float4* __restrict__ T, const float4* __restrict__ S,
+                                      float3 camera, float3 view, float3 point, float3 sun,
+                                      float3& rad, float3& trans, float shadow_length = 0.0f) {
     float r = sqrtf(dot3(camera, camera));
     float rmu = dot3(camera, view);
     float dtop = -rmu - sqrtf(rmu * rmu - r * r + P.top * P.top);
@@ -294,7 +294,7 @@ __device__ void sky_radiance_to_point(const DevParams& P, const SkyLut& L,
     bool ground = ray_intersects_ground<float>(P, r, mu);
     trans = lut_segment(L, T, r, mu, d, ground);
     float3 mie;
-    float4 sc = combined_scattering<H>(P, L, S, r, mu, mu_s, nu, ground, mie);
+    float4 sc = combined_scattering<H>(L, S, r, mu, mu_s, nu, ground, mie);
     if (!isinf(d)) {
         // Eq. (17): the second lookup at d - l, attenuated by T(x, x_{d-l}).
         float3 st = trans;
@@ -306,7 +306,7 @@ __device__ void sky_radiance_to_point(const DevParams& P, const SkyLut& L,
         float mu_p = (r * mu + d) / r_p;
         float mu_s_p = (r * mu_s + d * nu) / r_p;
         float3 mie_p;
-        float4 sc_p = combined_scattering<H>(P, L, S, r_p, mu_p, mu_s_p, nu, ground, mie_p);
+        float4 sc_p = combined_scattering<H>(L, S, r_p, mu_p, mu_s_p, nu, ground, mie_p);
         sc.x = sc.x - st.x * sc_p.x;
         sc.y = sc.y - st.y * sc_p.y;
         sc.z = sc.z - st.z * sc_p.z;
@@ -456,8 +456,8 @@ __device__ __forceinline__ float4 slice_scattering(const SliceConsts& C,
 // sky_radiance for a camera inside the atmosphere (so no move to the top
 // boundary), from the block's slice at the camera's r and mu_s.  Every
 // lookup coordinate is the reference's expression in the same binary32
-// operations, rounded the same (IEEE square roots; quotients by a per-frame
-// denominator through div_rn, bit for bit the IEEE quotient): the ground
+// operations, rounded the same (the square roots and the quotients by a
+// per-frame denominator bit for bit the IEEE ones): the ground
 // test switches between the two halves of the scattering texture, a ray
 // distance is a difference of two ~r-sized terms (down from 0.5 km: d = 0.5
 // from terms near 6360), and near the horizon the LUTs change steeply
@@ -488,9 +488,10 @@ __device__ void sky_radiance_slice(const DevParams& P, const SliceConsts& C,
 }
 
 // Draws of fewer pixels look the LUTs up directly: the slice costs a launch
-// and a stream-ordered allocation.  us per draw, slice / direct: 640x360 23.9 /
-// 15.9, 1280x720 38.4 / 36.2, 1920x1080 62.9 / 69.4 (binary16 53.6 / 70.6),
-// 3840x2160 190 / 230.
+// and a stream-ordered allocation.  us per draw, slice / direct: 640x360 27.9 /
+// 14.9, 1280x720 37.3 / 33.6, 1600x900 47.0 / 46.5, 1920x1080 59.3 / 62.2,
+// 3840x2160 182 / 220 (binary16 28.0 / 14.7, 34.6 / 35.8, 43.5 / 50.1, 53.4 /
+// 66.6, 161 / 237).
 constexpr size_t kDrawSliceMinPixels = 1500000;
 
 struct DrawArgs {
@@ -560,11 +561,12 @@ __global__ __launch_bounds__(256) void k_draw_slice(DevParams P, const float4* _
 // k_render_sky for a camera inside the atmosphere: every pixel starts at the
 // camera's r and mu_s, so the lookups there read the draw's slice (4 + 2 taps
 // from a table that fits the L1, not 16 + 4 from the LUTs, and no r and mu_s
-// coordinates), and a pixel with no geometry (depth 0) needs no others.
-// Bound by arithmetic and its latency (813 VALU instructions per pixel, 4 waves
-// per SIMD; 36 bytes of a pixel's traffic would take 15 us at 1080p): 54 us,
-// 101 us with IEEE divisions and square roots throughout and both lookups from
-// the LUTs.
+// coordinates), and a pixel with no geometry (depth 0) needs only the
+// transmittance's far end besides.
+// Bound by arithmetic and its latency (932 VALU instructions per wavefront, 3.6
+// wavefronts per SIMD, issue at 0.43 of the peak; 36 bytes of a pixel's traffic
+// would take 15 us at 1080p): 64 us a draw, 99 us with the compiler's divisions
+// and square roots throughout and both lookups from the LUTs.
 // smooth: smoothstep(0, 0.01, mu_s) (render_sky.h:182).
 template <bool H>
 __global__ __launch_bounds__(256) void k_render_sky_slice(
@@ -619,7 +621,7 @@ __global__ __launch_bounds__(256) void k_render_sky_slice(
                 tr);
 }
 
-// Bound by the texture path of its scattered taps (TA busy 0.9 of the time):
+// Bound by the texture path of its scattered taps (TA busy 0.8 of the time):
 // with binary16 LUTs the two x neighbours of a tap pair come in one load, 8
 // instead of 16 per ray (4M random rays 242 -> 181 us).
 template <bool H>
@@ -825,7 +827,7 @@ __device__ void render_frame_block(const DevParams& P, const float4* __restrict_
     const FrameView v = frame_view(P, alt, zs);
     const float3 cam = v.cam, sun = v.sun;
     const float r = v.r;
-    const SkyLut L = sky_lut(P);
+    SkyLut L;
     SliceConsts sc;
     if constexpr (SLICE) {
         if (frame_slice) {
@@ -836,6 +838,8 @@ __device__ void render_frame_block(const DevParams& P, const float4* __restrict_
         }
         sc = slice_consts(P, r);
         __syncthreads();
+    } else {
+        L = sky_lut(P);
     }
     const uint32_t fk = ray_frame_key(seed, frame);
     static_assert(kFramePixelsPerThread % kRayGroup == 0);
