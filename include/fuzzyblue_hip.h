@@ -431,7 +431,14 @@ typedef struct fb_draw_parameters {
  * float per pixel (the subpassInput depth, render_sky.frag:26), or NULL for
  * an infinitely distant background (reverse-Z depth 0).  color and
  * transmittance: device float4 per pixel, row-major, row 0 = top (Vulkan
- * framebuffer origin).  transmittance may be NULL when compositing. */
+ * framebuffer origin).  transmittance may be NULL when compositing.
+ *
+ * A draw of at least 1.5 M pixels with the camera in the atmosphere evaluates
+ * the LUTs at the camera's altitude and the sun's angle first, into
+ * stream-ordered scratch on `stream` (16 bytes x ((NU + 1) MU + transmittance
+ * mu), 22.5 KB at default sizes), freed after the launch; where that cannot be
+ * had, or the stream is captured, it looks the LUTs up per pixel, as smaller
+ * draws do.  The two agree up to the order of rounding of an interpolation. */
 fb_status fb_render_sky(fb_builder *b, fb_stream stream, const fb_atmosphere *a,
                         const fb_draw_parameters *draw, const float *depth,
                         uint32_t width, uint32_t height, float *color,
