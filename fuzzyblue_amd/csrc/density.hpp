@@ -56,7 +56,7 @@ struct DenRow {
     // peak an ulp of it counts: rounding sin(theta) omega.x once for the whole
     // row, as FP32 mode does, raises a g = 0.95 density's error by 14%.
     __device__ __forceinline__ float nu2(int m) const {
-        return fmaf(sizeof(G) == sizeof(double) ? cx[m] : c_den_phi[m].x, omx, omzc);
+        return fmaf(sizeof(G) == sizeof(double) ? cx[m] : c_den.phi[m].x, omx, omzc);
     }
 };
 // Block constants of the quadrature.
@@ -131,7 +131,7 @@ __device__ __forceinline__ void density_row(const DenConst& k, const DenTexel* d
     }
 #pragma unroll
     for (int m = 0; m < kDenPhi / 2; ++m) {
-        const float cp = c_den_phi[m].x, sp = c_den_phi[m].y;
+        const float cp = c_den.phi[m].x, sp = c_den.phi[m].y;
         float q, qw;
         const float3 p = den_phase(k, row.nu2(m), q, qw);
         if (MOM) {
@@ -174,7 +174,7 @@ __device__ __forceinline__ void density_kink(const DenConst& k, const DenTexel* 
     const float c = row.c - kink.w;
 #pragma unroll 4
     for (int m = 0; m < kDenPhi / 2; ++m) {
-        const float cp = c_den_phi[m].x, sp = c_den_phi[m].y;
+        const float cp = c_den.phi[m].x, sp = c_den.phi[m].y;
         float q, qw;
         (void)den_phase(k, row.nu2(m), q, qw);
 #pragma unroll
@@ -211,7 +211,7 @@ __device__ __forceinline__ void density_ground(const DenConst& k, const DenTexel
     }
 #pragma unroll 4
     for (int m = 0; m < kDenPhi / 2; ++m) {
-        const float cp = c_den_phi[m].x, sp = c_den_phi[m].y;
+        const float cp = c_den.phi[m].x, sp = c_den.phi[m].y;
         float q, qw;
         const float3 p = den_phase(k, row.nu2(m), q, qw);
 #pragma unroll
@@ -342,12 +342,12 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
     }
     __syncthreads();
     if (ground_lane) {
-        const float ct = c_den_cos[gl0];
+        const float ct = c_den.cos[gl0];
         const float C = ct * osz;
         // Entry coordinate of the lookup (slot k at entry k + 1): ec + e1 (nu1 - C).
         const float ec = fmaf((rf + ct * gd.w) * ginv * osz, hE, hE + 1.0f);
         const float e1 = gd.w * ginv * hE;
-        const float e_half = e1 * c_den_sin[gl0] * sin_s;
+        const float e_half = e1 * c_den.sin[gl0] * sin_s;
         int knots = -1;
         float4 lin = make_float4(0.0f, 0.0f, 0.0f, e1), slope = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float4 kink = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -417,7 +417,7 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
         } else {
             const float4 gl = s_glin[row], gs = s_gslope[row];
             const float h = 1.0f / kc.hnu;
-            const float dn = fmaf(float(k) - kc.hnu1, h, -c_den_cos[row] * osz);  // nu1 - centre
+            const float dn = fmaf(float(k) - kc.hnu1, h, -c_den.cos[row] * osz);  // nu1 - centre
             const float3 d = make_float3(fmaf(gs.x, h, w.x - v.x), fmaf(gs.y, h, w.y - v.y),
                                          fmaf(gs.z, h, w.z - v.z));
             ProfEntry p;
@@ -442,9 +442,9 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
         DenRow<G> row;
         row.c = SINGLE ? ct * osz : fmaf(ct * osz, kc.hnu, kc.hnu1);
         row.omzc = ct * omz;
-        row.st = c_den_sin[l];
+        row.st = c_den.sin[l];
         row.omx = OUTER ? omx : row.st * omx;
-        row.cx = c_den_cx + l * kDenPhi / 2;
+        row.cx = c_den.cx + l * kDenPhi / 2;
         row.pr = s_prof + l * nent;
         row.pp = s_pair + l * nent;
         return row;
@@ -460,7 +460,7 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
     if (OUTER && (bx + 1) * int(blockDim.x) > lay.inner) {
         for (int e = tid; e < kDenTheta * kDenPhi / 2; e += blockDim.x) {
             const int l = e / (kDenPhi / 2), m = e % (kDenPhi / 2);
-            const float4 o = c_den_dir[l * kDenPhi + m];
+            const float4 o = c_den.dir[l * kDenPhi + m];
             const DenRow<G> row = make_row(l, o.z, 0.0f, 0.0f);
             const float dn = o.x * sin_s;  // nu1 - centre
             float3 L;
@@ -543,7 +543,7 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
         texel_setup(0, y, dt);
         float3 lo = make_float3(0.0f, 0.0f, 0.0f), hi = lo;  // azimuth pi, 0
         for (int l = l0; l < kDenTheta; l += S) {
-            const float4 d0 = c_den_dir[l * kDenPhi];
+            const float4 d0 = c_den.dir[l * kDenPhi];
             const DenRow<G> row = make_row(l, d0.z, dt.omx, dt.omz);
             float3 a = make_float3(0.0f, 0.0f, 0.0f), b = a;
 #pragma unroll
@@ -576,7 +576,7 @@ __device__ __forceinline__ void scattering_density_block(const DevParams& P, con
 #pragma unroll
     for (int u = 0; u < TPX; ++u) acc[u] = make_float3(0.0f, 0.0f, 0.0f);
     for (int l = l0; l < kDenTheta; l += S) {
-        const float4 d0 = c_den_dir[l * kDenPhi];
+        const float4 d0 = c_den.dir[l * kDenPhi];
         const float ct = d0.z, dom = d0.w;
         const DenRow<G> row = make_row(l, ct, dt[0].omx, dt[0].omz);
         float3 a[TPX], m0 = make_float3(0.0f, 0.0f, 0.0f), m1 = m0;

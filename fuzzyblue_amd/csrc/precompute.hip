@@ -19,33 +19,36 @@ namespace fbk {
 // Direction tables of the irradiance quadrature, as the density's
 // (precompute_device.hpp): j = 0..15 (theta), i = 0..63 (phi), dtheta = dphi
 // = pi/32 (indirect_irradiance.comp:20-33).
-__constant__ float4 c_ind_dir[kIndTheta * kIndPhi];
-__constant__ float c_ind_cos[kIndTheta];
-__constant__ double c_ind_cos_d[kIndTheta];
+struct IrradianceTables {
+    float4 dir[kIndTheta * kIndPhi];
+    float cos[kIndTheta];
+    double cos_d[kIndTheta];
+
+    static IrradianceTables make() {
+        IrradianceTables t;
+        const float PI = 3.14159265358979323846f;
+        const float dphi = PI / float(32), dtheta = PI / float(32);
+        const double dtheta_d = M_PI / 32.0;
+        for (int j = 0; j < kIndTheta; ++j) {
+            const float theta = (float(j) + 0.5f) * dtheta;
+            t.cos[j] = cosf(theta);
+            t.cos_d[j] = ::cos((double(j) + 0.5) * dtheta_d);
+            for (int i = 0; i < kIndPhi; ++i) {
+                const float phi = (float(i) + 0.5f) * dphi;
+                const float domega = dtheta * dphi * sinf(theta);
+                t.dir[j * kIndPhi + i] = make_float4(cosf(phi) * sinf(theta),
+                                                     sinf(phi) * sinf(theta), cosf(theta), domega);
+            }
+        }
+        return t;
+    }
+};
+__constant__ IrradianceTables c_ind;
 
 hipError_t upload_tables() {
-    static float4 ind[kIndTheta * kIndPhi];
-    static float icos[kIndTheta];
-    static double icos_d[kIndTheta];
-    const float PI = 3.14159265358979323846f;
-    const float dphi = PI / float(32), dtheta = PI / float(32);
-    const double dtheta_d = M_PI / 32.0;
-    for (int j = 0; j < kIndTheta; ++j) {
-        float theta = (float(j) + 0.5f) * dtheta;
-        icos[j] = cosf(theta);
-        icos_d[j] = cos((double(j) + 0.5) * dtheta_d);
-        for (int i = 0; i < kIndPhi; ++i) {
-            float phi = (float(i) + 0.5f) * dphi;
-            float domega = dtheta * dphi * sinf(theta);
-            ind[j * kIndPhi + i] =
-                make_float4(cosf(phi) * sinf(theta), sinf(phi) * sinf(theta), cosf(theta), domega);
-        }
-    }
-    hipError_t e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_ind_dir), ind, sizeof(ind))) != hipSuccess) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_ind_cos), icos, sizeof(icos))) != hipSuccess) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_ind_cos_d), icos_d, sizeof(icos_d))) != hipSuccess)
-        return e;
+    static const IrradianceTables t = IrradianceTables::make();
+    hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_ind), &t, sizeof(t));
+    if (e != hipSuccess) return e;
     // Each translation unit that reads the density tables has its own.
     if ((e = upload_density_tables()) != hipSuccess) return e;
     if ((e = DensityLaunch<float>::upload()) != hipSuccess) return e;
@@ -55,9 +58,9 @@ hipError_t upload_tables() {
 template <typename G>
 __device__ __forceinline__ G ind_cos(int j);
 template <>
-__device__ __forceinline__ float ind_cos<float>(int j) { return c_ind_cos[j]; }
+__device__ __forceinline__ float ind_cos<float>(int j) { return c_ind.cos[j]; }
 template <>
-__device__ __forceinline__ double ind_cos<double>(int j) { return c_ind_cos_d[j]; }
+__device__ __forceinline__ double ind_cos<double>(int j) { return c_ind.cos_d[j]; }
 
 // Running sum with optional Neumaier compensation (precision mode).
 template <bool COMP>
@@ -728,7 +731,7 @@ __device__ __forceinline__ void density_geometry_block(const DevParams& P, const
                                  tg.y * P.albedo[1] * (1.0f / kPi),
                                  tg.z * P.albedo[2] * (1.0f / kPi), float(dg));
                 // The ground normal's length does not depend on phi.
-                const float4 o = c_den_dir[l * kDenPhi];
+                const float4 o = c_den.dir[l * kDenPhi];
                 const G st2 = G(o.x) * G(o.x) + G(o.y) * G(o.y);
                 const G gz = r + ct * dg;
                 ginv = float(G(1) / sqrt(st2 * dg * dg + gz * gz));
@@ -814,7 +817,7 @@ __device__ __forceinline__ void indirect_irradiance_block(const DevParams& P, co
     const int kmax = NU - 1;
     float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
     for (int jj = 0; jj < kIndTheta; ++jj) {
-        const float4 om = c_ind_dir[jj * kIndPhi + lane];
+        const float4 om = c_ind.dir[jj * kIndPhi + lane];
         const float nu = fmaf(om.x, osx, om.z * osz);
         const float t = fmaf(nu, hnu, hnu);
         float3 v = prof_lerp(s_prof + jj * nent, t, kmax);

@@ -24,52 +24,52 @@ namespace fbk {
 // Direction tables of the density quadrature, computed once on the host in
 // binary32 exactly as the reference evaluates them (scattering_density.comp:
 // 34-66), and in binary64 for the precision mode's geometry: l = 0..15
-// (theta), m = 0..31 (phi), dtheta = dphi = pi/16.  One copy per translation
-// unit (upload_density_tables in each).
-static __constant__ float4 c_den_dir[kDenTheta * kDenPhi];  // (cos phi sin t, sin phi sin t, cos t, domega)
-static __constant__ float c_den_cos[kDenTheta];
-static __constant__ float c_den_sin[kDenTheta];
-static __constant__ float2 c_den_phi[kDenPhi / 2];  // cos phi, sin phi of the half turn m < 16
-static __constant__ float c_den_cx[kDenTheta * kDenPhi / 2];  // c_den_dir's x of the half turn
-static __constant__ double c_den_cos_d[kDenTheta];
+// (theta), m = 0..31 (phi), dtheta = dphi = pi/16.  One symbol, so that a
+// builder uploads it with one copy, in each translation unit that reads it.
+struct DensityTables {
+    float4 dir[kDenTheta * kDenPhi];     // (cos phi sin t, sin phi sin t, cos t, domega)
+    float2 phi[kDenPhi / 2];             // cos phi, sin phi of the half turn m < 16
+    float cx[kDenTheta * kDenPhi / 2];   // dir's x of the half turn
+    float cos[kDenTheta], sin[kDenTheta];
+    double cos_d[kDenTheta];
+
+    static DensityTables make() {
+        DensityTables t;
+        const float PI = 3.14159265358979323846f;
+        const float dphi = PI / float(16), dtheta = PI / float(16);
+        const double dtheta_d = M_PI / 16.0;
+        for (int l = 0; l < kDenTheta; ++l) {
+            const float theta = (float(l) + 0.5f) * dtheta;
+            const float ct = cosf(theta), st = sinf(theta);
+            t.cos[l] = ct;
+            t.sin[l] = st;
+            t.cos_d[l] = ::cos((double(l) + 0.5) * dtheta_d);
+            for (int m = 0; m < kDenPhi; ++m) {
+                const float phi = (float(m) + 0.5f) * dphi;
+                const float domega = dtheta * dphi * sinf(theta);
+                t.dir[l * kDenPhi + m] = make_float4(cosf(phi) * st, sinf(phi) * st, ct, domega);
+                if (m < kDenPhi / 2) {
+                    t.phi[m] = make_float2(cosf(phi), sinf(phi));
+                    t.cx[l * kDenPhi / 2 + m] = t.dir[l * kDenPhi + m].x;
+                }
+            }
+        }
+        return t;
+    }
+};
+static __constant__ DensityTables c_den;
 
 static hipError_t upload_density_tables() {
-    float4 den[kDenTheta * kDenPhi];
-    float2 phis[kDenPhi / 2];
-    float dcos[kDenTheta], dsin[kDenTheta], cx[kDenTheta * kDenPhi / 2];
-    double dcos_d[kDenTheta];
-    const float PI = 3.14159265358979323846f;
-    const float dphi = PI / float(16), dtheta = PI / float(16);
-    const double dtheta_d = M_PI / 16.0;
-    for (int l = 0; l < kDenTheta; ++l) {
-        float theta = (float(l) + 0.5f) * dtheta;
-        float ct = cosf(theta), st = sinf(theta);
-        dcos[l] = ct;
-        dsin[l] = st;
-        dcos_d[l] = cos((double(l) + 0.5) * dtheta_d);
-        for (int m = 0; m < kDenPhi; ++m) {
-            float phi = (float(m) + 0.5f) * dphi;
-            if (m < kDenPhi / 2) phis[m] = make_float2(cosf(phi), sinf(phi));
-            float domega = dtheta * dphi * sinf(theta);
-            den[l * kDenPhi + m] = make_float4(cosf(phi) * st, sinf(phi) * st, ct, domega);
-            if (m < kDenPhi / 2) cx[l * kDenPhi / 2 + m] = den[l * kDenPhi + m].x;
-        }
-    }
-    hipError_t e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_dir), den, sizeof(den))) != hipSuccess) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_cos), dcos, sizeof(dcos))) != hipSuccess) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_sin), dsin, sizeof(dsin))) != hipSuccess) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_phi), phis, sizeof(phis))) != hipSuccess) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_den_cx), cx, sizeof(cx))) != hipSuccess) return e;
-    return hipMemcpyToSymbol(HIP_SYMBOL(c_den_cos_d), dcos_d, sizeof(dcos_d));
+    static const DensityTables t = DensityTables::make();
+    return hipMemcpyToSymbol(HIP_SYMBOL(c_den), &t, sizeof(t));
 }
 
 template <typename G>
 __device__ __forceinline__ G den_cos(int l);
 template <>
-__device__ __forceinline__ float den_cos<float>(int l) { return c_den_cos[l]; }
+__device__ __forceinline__ float den_cos<float>(int l) { return c_den.cos[l]; }
 template <>
-__device__ __forceinline__ double den_cos<double>(int l) { return c_den_cos_d[l]; }
+__device__ __forceinline__ double den_cos<double>(int l) { return c_den.cos_d[l]; }
 
 // ------------------------------------------------------------ nu profiles
 template <typename G>

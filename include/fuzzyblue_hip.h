@@ -437,8 +437,9 @@ typedef struct fb_draw_parameters {
  * the LUTs at the camera's altitude and the sun's angle first, into
  * stream-ordered scratch on `stream` (16 bytes x ((NU + 1) MU + transmittance
  * mu), 22.5 KB at default sizes), freed after the launch; where that cannot be
- * had, or the stream is captured, it looks the LUTs up per pixel, as smaller
- * draws do.  The two agree up to the order of rounding of an interpolation. */
+ * had (or not without entering a capture, as on the legacy stream while a
+ * blocking stream is captured) it looks the LUTs up per pixel, as smaller draws
+ * do.  The two agree up to the order of rounding of an interpolation. */
 fb_status fb_render_sky(fb_builder *b, fb_stream stream, const fb_atmosphere *a,
                         const fb_draw_parameters *draw, const float *depth,
                         uint32_t width, uint32_t height, float *color,
